@@ -540,6 +540,8 @@ class World {
                 (void)hipHostFree(c.p);
             }
             for (auto &e : ring_) (void)hipEventDestroy(e);
+            for (auto &e : read_ev_)
+                if (e) (void)hipEventDestroy(e);
             if (side_) {
                 (void)hipStreamSynchronize(side_);
                 (void)hipEventDestroy(fork_);
@@ -744,6 +746,98 @@ class World {
         return NXM_OK;
     }
 
+    // A host array that a readback fills: rows of `comps` words by id.
+    struct ReadItem {
+        int plane, comps;
+        void *dst;
+    };
+
+    // Reads rows of the scene's particles in id order: gathered on the device into the arena
+    // that the next step will write (its position planes stay: the canonical sort reads
+    // them), then copied through two pinned chunks, one being filled while the other is
+    // taken (copy_out).  At most 33 words a particle.  Synchronizes; the errors latched so
+    // far are reported before anything is written.
+    nxm_status read_rows(nxm_scene *sc, std::initializer_list<ReadItem> items)
+    {
+        HIP_TRY(hipSetDevice(ctx_->device));
+        const size_t n = sc->hp.n;
+        ReadList list{};
+        std::vector<std::pair<char *, size_t>> parts;   // destinations, in the gathered order
+        size_t words = 0;
+        for (const ReadItem &it : items) {
+            if (!it.dst || n == 0) continue;
+            list.rows[list.n++] = ReadRows{it.plane, it.comps, words};
+            parts.emplace_back(static_cast<char *>(it.dst), 4 * n * it.comps);
+            words += n * it.comps;
+        }
+        if (words == 0) return sync();
+        if (words > (size_t)(NUM_PLANES - PVX) * p_cap_) return fail(NXM_ERR_INVALID_ARGUMENT, "readback too wide");
+        float *dev = arena(cur_ ^ 1).plane(PVX);
+        for (const SceneRange &r : sc->ranges)
+            launch_read_rows(arena(cur_), r.start, r.count, list, dev, (int)ctx_->num_cus * 8, stream_);
+        HIP_TRY(hipGetLastError());
+        return copy_out(dev, parts);
+    }
+
+    // Copies consecutive device bytes to the host destinations, in order (read_rows).
+    nxm_status copy_out(const float *dev, const std::vector<std::pair<char *, size_t>> &parts)
+    {
+        size_t total = 0;
+        for (auto &d : parts) total += d.second;
+        // Pinned staging of the context's pool, one size for every read: two halves, then the
+        // slots' error counters.
+        const size_t nslots = std::min(slots_.size(), ctr_.n);
+        int held = -1;
+        char *pin = nullptr;
+        HIP_TRY(ctx_->pool.take(2 * READ_CHUNK + MAX_SCENES * sizeof(SceneCtr), &held, &pin));
+        nxm_status st = copy_through(pin, reinterpret_cast<const char *>(dev), total, parts, nslots);
+        if (st != NXM_OK) (void)hipStreamSynchronize(stream_);   // nothing still writes the chunk
+        HIP_TRY(ctx_->pool.give(held, nullptr));
+        return st;
+    }
+
+    nxm_status copy_through(char *pin, const char *dev, size_t total, const std::vector<std::pair<char *, size_t>> &parts,
+                            size_t nslots)
+    {
+        for (auto &e : read_ev_)
+            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        const size_t chunk = READ_CHUNK;
+        SceneCtr *errs = reinterpret_cast<SceneCtr *>(pin + 2 * chunk);
+        if (nslots) HIP_TRY(hipMemcpyAsync(errs, ctr_.p, nslots * sizeof(SceneCtr), hipMemcpyDeviceToHost, stream_));
+        auto queue = [&](size_t at, int k) -> hipError_t {
+            hipError_t e = hipMemcpyAsync(pin + k * chunk, dev + at, std::min(chunk, total - at), hipMemcpyDeviceToHost, stream_);
+            return e != hipSuccess ? e : hipEventRecord(read_ev_[k], stream_);
+        };
+        HIP_TRY(queue(0, 0));
+        size_t part = 0, done = 0;   // destination being filled and its bytes so far
+        int k = 0;
+        for (size_t at = 0; at < total; at += chunk, k ^= 1) {
+            if (at + chunk < total) HIP_TRY(queue(at + chunk, k ^ 1));
+            HIP_TRY(hipEventSynchronize(read_ev_[k]));
+            if (at == 0) {
+                nxm_status st = note_errors(errs, nslots);
+                if (st != NXM_OK) return st;
+            }
+            const size_t got = std::min(chunk, total - at);
+            for (size_t used = 0; used < got;) {
+                const size_t m = std::min(got - used, parts[part].second - done);
+                std::memcpy(parts[part].first + done, pin + k * chunk + used, m);
+                used += m;
+                done += m;
+                if (done == parts[part].second) { ++part; done = 0; }
+            }
+        }
+        return NXM_OK;
+    }
+
+    // Particle state in id order into arrays of the caller's (any may be null).
+    nxm_status read_state(nxm_scene *sc, float *x, float *v, float *C, float *F, float *mass, float *vol0, float *pstate,
+                          uint32_t *flags)
+    {
+        return read_rows(sc, {{PX, 3, x}, {PVX, 3, v}, {PC0, 9, C}, {PF0, 9, F}, {PMASS, 1, mass}, {PVOL0, 1, vol0},
+                              {PS0, 3, pstate}, {PFLAGS, 1, flags}});
+    }
+
     // Reads the scene's particle state into its host arrays (id order).
     nxm_status pull(nxm_scene *sc)
     {
@@ -751,70 +845,28 @@ class World {
         if (st == NXM_OK) st = pull_clock(sc);
         if (st != NXM_OK) return st;
         HostParticles &hp = sc->hp;
-        Arena a = arena(cur_);
-        std::vector<float> buf;
-        std::vector<uint32_t> ids, fl;
-        for (const SceneRange &r : sc->ranges) {
-            buf.resize(r.count);
-            ids.resize(r.count);
-            fl.resize(r.count);
-            HIP_TRY(hipMemcpy(ids.data(), a.uplane(PID) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-            HIP_TRY(hipMemcpy(fl.data(), a.uplane(PFLAGS) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-            for (uint32_t i = 0; i < r.count; ++i) {
-                hp.enabled[ids[i]] = (fl[i] & FLAG_ENABLED) ? 1u : 0u;
-                hp.fixed[ids[i]] = (fl[i] & FLAG_FIXED) ? 1u : 0u;
-            }
-            auto get = [&](int p, float *dst, int stride, int comp) -> hipError_t {
-                hipError_t e = hipMemcpy(buf.data(), a.plane(p) + r.start, r.count * 4, hipMemcpyDeviceToHost);
-                if (e != hipSuccess) return e;
-                for (uint32_t i = 0; i < r.count; ++i) dst[(size_t)ids[i] * stride + comp] = buf[i];
-                return hipSuccess;
-            };
-            for (int c = 0; c < 3; ++c) HIP_TRY(get(PX + c, hp.x.data(), 3, c));
-            for (int c = 0; c < 3; ++c) HIP_TRY(get(PVX + c, hp.v.data(), 3, c));
-            for (int c = 0; c < 9; ++c) HIP_TRY(get(PC0 + c, hp.C.data(), 9, c));
-            for (int c = 0; c < 9; ++c) HIP_TRY(get(PF0 + c, hp.F.data(), 9, c));
-            HIP_TRY(get(PMASS, hp.mass.data(), 1, 0));
-            HIP_TRY(get(PVOL0, hp.vol0.data(), 1, 0));
+        std::vector<uint32_t> fl(hp.n);
+        std::vector<float> ps(3 * hp.n);
+        st = read_state(sc, hp.x.data(), hp.v.data(), hp.C.data(), hp.F.data(), hp.mass.data(), hp.vol0.data(), ps.data(),
+                        fl.data());
+        if (st != NXM_OK) return st;
+        for (size_t i = 0; i < hp.n; ++i) {
+            hp.enabled[i] = (fl[i] & FLAG_ENABLED) ? 1u : 0u;
+            hp.fixed[i] = (fl[i] & FLAG_FIXED) ? 1u : 0u;
             // plastic state: the sand tags carry three words, snow one
-            std::vector<float> ps(3 * (size_t)r.count);
-            for (int c = 0; c < 3; ++c) {
-                HIP_TRY(hipMemcpy(buf.data(), a.plane(PS0 + c) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-                for (uint32_t i = 0; i < r.count; ++i) {
-                    uint32_t id = ids[i];
-                    if (c < pstate_words(hp.tag[id])) hp.pstate[3 * (size_t)id + c] = buf[i];
-                }
-            }
-            if (sc->cpic) {
-                HIP_TRY(hipMemcpy(buf.data(), a.plane(PAFF) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-                for (uint32_t i = 0; i < r.count; ++i) std::memcpy(&hp.aff[ids[i]], &buf[i], 4);
-                for (int c = 0; c < 4; ++c) HIP_TRY(get(PNX + c, hp.cdf.data(), 4, c));
-                // An empty affinity means a zero contact field; the device does not store it.
-                for (uint32_t i = 0; i < r.count; ++i)
-                    if (hp.aff[ids[i]] == 0u) std::fill(&hp.cdf[4 * (size_t)ids[i]], &hp.cdf[4 * (size_t)ids[i] + 4], 0.0f);
-            }
+            for (int c = 0; c < pstate_words(hp.tag[i]); ++c) hp.pstate[3 * i + c] = ps[3 * i + c];
+        }
+        if (sc->cpic) {
+            st = read_rows(sc, {{PAFF, 1, hp.aff.data()}, {PNX, 4, hp.cdf.data()}});
+            if (st != NXM_OK) return st;
+            // An empty affinity means a zero contact field; the device does not store it.
+            for (size_t i = 0; i < hp.n; ++i)
+                if (hp.aff[i] == 0u) std::fill(&hp.cdf[4 * i], &hp.cdf[4 * i + 4], 0.0f);
         }
         return NXM_OK;
     }
 
-    nxm_status positions(nxm_scene *sc, float *xyz)
-    {
-        nxm_status st = sync();
-        if (st != NXM_OK) return st;
-        Arena a = arena(cur_);
-        std::vector<float> buf;
-        std::vector<uint32_t> ids;
-        for (const SceneRange &r : sc->ranges) {
-            buf.resize(r.count);
-            ids.resize(r.count);
-            HIP_TRY(hipMemcpy(ids.data(), a.uplane(PID) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-            for (int c = 0; c < 3; ++c) {
-                HIP_TRY(hipMemcpy(buf.data(), a.plane(PX + c) + r.start, r.count * 4, hipMemcpyDeviceToHost));
-                for (uint32_t i = 0; i < r.count; ++i) xyz[3 * (size_t)ids[i] + c] = buf[i];
-            }
-        }
-        return NXM_OK;
-    }
+    nxm_status positions(nxm_scene *sc, float *xyz) { return read_rows(sc, {{PX, 3, xyz}}); }
 
     // Enqueues one substep of every active scene.
     nxm_status step(nxm_stage_times *times)
@@ -1013,26 +1065,25 @@ class World {
         const size_t n = sc->hp.n;
         if (n == 0) return NXM_OK;
         const HostParticles &hp = sc->hp;
-        DevBuf<uint32_t> group;
-        DevBuf<float> props, dout;
-        DevBuf<float4> pal;
-        HIP_TRY(group.reserve(n));
-        HIP_TRY(props.reserve(2 * n));
-        HIP_TRY(pal.reserve(npal));
-        HIP_TRY(dout.reserve(24 * n));
-        nxm_status st = put_async(group.p, hp.group.data(), n * 4);
-        if (st == NXM_OK) st = put_async(props.p, hp.phase.data(), n * 4);
-        if (st == NXM_OK) st = put_async(props.p + n, hp.radius.data(), n * 4);
-        if (st == NXM_OK) st = put_async(pal.p, palette, (size_t)npal * 16);
+        // The records and the constant properties they use lie in the arena that the next
+        // step will write, as in read_rows (24 + 3 words a particle).
+        float *dout = arena(cur_ ^ 1).plane(PVX), *props = dout + 24 * n;
+        uint32_t *group = reinterpret_cast<uint32_t *>(props + 2 * n);
+        if (npal > read_palette_.n) {
+            nxm_status st = sync();   // a call in flight may read the one that is replaced
+            if (st != NXM_OK) return st;
+            HIP_TRY(read_palette_.reserve(npal));
+        }
+        nxm_status st = put_async(group, hp.group.data(), n * 4);
+        if (st == NXM_OK) st = put_async(props, hp.phase.data(), n * 4);
+        if (st == NXM_OK) st = put_async(props + n, hp.radius.data(), n * 4);
+        if (st == NXM_OK) st = put_async(read_palette_.p, palette, (size_t)npal * 16);
         if (st != NXM_OK) return st;
         for (const SceneRange &r : sc->ranges)
-            launch_prep_readback(arena(cur_), r.start, r.count, group.p, props.p, props.p + n, pal.p, npal, mode, sc->h,
-                                 sc->dt, sc->cpic, dout.p, (int)ctx_->num_cus * 8, stream_);
+            launch_prep_readback(arena(cur_), r.start, r.count, group, props, props + n, read_palette_.p, npal, mode, sc->h,
+                                 sc->dt, sc->cpic, dout, (int)ctx_->num_cus * 8, stream_);
         HIP_TRY(hipGetLastError());
-        st = sync();
-        if (st != NXM_OK) return st;
-        HIP_TRY(hipMemcpy(out, dout.p, 24 * n * sizeof(float), hipMemcpyDeviceToHost));
-        return NXM_OK;
+        return copy_out(dout, {{reinterpret_cast<char *>(out), 96 * n}});
     }
 
     // ---- inspection of the last step ----
@@ -1521,6 +1572,12 @@ class World {
         if (nslots == 0 || !ctr_.p) return NXM_OK;
         std::vector<SceneCtr> c(nslots);
         HIP_TRY(hipMemcpy(c.data(), ctr_.p, c.size() * sizeof(SceneCtr), hipMemcpyDeviceToHost));
+        return note_errors(c.data(), nslots);
+    }
+
+    // Takes the error bits of the slots' counters c to their scenes, and clears them.
+    nxm_status note_errors(const SceneCtr *c, size_t nslots)
+    {
         nxm_status first = NXM_OK;
         bool any = false;
         for (uint32_t i = 0; i < nslots; ++i) {
@@ -1529,7 +1586,7 @@ class World {
             if (slots_[i].scene) slots_[i].scene->error |= c[i].err;
         }
         if (any) {
-            HIP_TRY(hipMemset(ctr_.p, 0, c.size() * sizeof(SceneCtr)));
+            HIP_TRY(hipMemset(ctr_.p, 0, nslots * sizeof(SceneCtr)));
             for (uint32_t i = 0; i < nslots; ++i) {
                 if (!c[i].err) continue;
                 if (first == NXM_OK) {
@@ -1716,6 +1773,9 @@ class World {
     std::vector<size_t> tune_slot_;
     std::vector<hipEvent_t> tune_ev_;
     std::vector<PinnedChunk> pins_;
+    static constexpr size_t READ_CHUNK = (size_t)4 << 20;
+    hipEvent_t read_ev_[2] = {};
+    DevBuf<float4> read_palette_;
     bool graph_on_ = false;
     uint64_t gen_ = 0;                 // bumped whenever a buffer address or table changes
     hipGraphExec_t gexec_[2] = {};     // one per arena parity
@@ -2308,31 +2368,40 @@ nxm_status nxm_scene_read_particles_soa(nxm_scene *sc, const nxm_particles_soa *
 {
     if (!sc || !o) return fail(NXM_ERR_INVALID_ARGUMENT, "null argument");
     if (n < sc->hp.n) return fail(NXM_ERR_INVALID_ARGUMENT, "output too small");
-    if (sc->world) {
-        nxm_status st = sc->world->pull(sc);
-        if (st != NXM_OK) return st;
-    }
     const HostParticles &hp = sc->hp;
-    size_t m = hp.n;
-    if (o->position) std::memcpy(o->position, hp.x.data(), m * 12);
-    if (o->velocity) std::memcpy(o->velocity, hp.v.data(), m * 12);
-    if (o->def_grad) std::memcpy(o->def_grad, hp.F.data(), m * 36);
-    if (o->affine) std::memcpy(o->affine, hp.C.data(), m * 36);
-    if (o->init_volume) std::memcpy(o->init_volume, hp.vol0.data(), m * 4);
+    const size_t m = hp.n;
+    const float *pstate = hp.pstate.data();
+    std::vector<float> ps;
+    if (sc->world) {
+        // The state straight into the caller's arrays; the host mirror stays as it is.
+        std::vector<uint32_t> fl(o->enabled || o->fixed ? m : 0);
+        if (o->model_data) ps.resize(3 * m);
+        nxm_status st = sc->world->read_state(sc, o->position, o->velocity, o->affine, o->def_grad, o->mass, o->init_volume,
+                                              o->model_data ? ps.data() : nullptr, fl.empty() ? nullptr : fl.data());
+        if (st != NXM_OK) return st;
+        if (o->enabled) for (size_t i = 0; i < m; ++i) o->enabled[i] = (fl[i] & FLAG_ENABLED) ? 1u : 0u;
+        if (o->fixed) for (size_t i = 0; i < m; ++i) o->fixed[i] = (fl[i] & FLAG_FIXED) ? 1u : 0u;
+        pstate = ps.data();
+    } else {
+        if (o->position) std::memcpy(o->position, hp.x.data(), m * 12);
+        if (o->velocity) std::memcpy(o->velocity, hp.v.data(), m * 12);
+        if (o->def_grad) std::memcpy(o->def_grad, hp.F.data(), m * 36);
+        if (o->affine) std::memcpy(o->affine, hp.C.data(), m * 36);
+        if (o->init_volume) std::memcpy(o->init_volume, hp.vol0.data(), m * 4);
+        if (o->mass) std::memcpy(o->mass, hp.mass.data(), m * 4);
+        if (o->enabled) std::memcpy(o->enabled, hp.enabled.data(), m * 4);
+        if (o->fixed) std::memcpy(o->fixed, hp.fixed.data(), m * 4);
+    }
     if (o->init_radius) std::memcpy(o->init_radius, hp.radius.data(), m * 4);
-    if (o->mass) std::memcpy(o->mass, hp.mass.data(), m * 4);
     if (o->damping) std::memcpy(o->damping, hp.damping.data(), m * 4);
     if (o->phase) std::memcpy(o->phase, hp.phase.data(), m * 4);
     if (o->boundary_friction) std::memcpy(o->boundary_friction, hp.bfric.data(), m * 4);
     if (o->group_id) std::memcpy(o->group_id, hp.group.data(), m * 4);
-    if (o->enabled) std::memcpy(o->enabled, hp.enabled.data(), m * 4);
-    if (o->fixed) std::memcpy(o->fixed, hp.fixed.data(), m * 4);
     if (o->model_tag) std::memcpy(o->model_tag, hp.tag.data(), m * 4);
     if (o->model_data) {
-        for (size_t i = 0; i < m; ++i) {
-            std::memcpy(o->model_data + 24 * i, &hp.words[24 * i], 96);
-            std::memcpy(o->model_data + 24 * i, &hp.pstate[3 * i], 4 * (size_t)pstate_words(hp.tag[i]));
-        }
+        std::memcpy(o->model_data, hp.words.data(), 96 * m);
+        for (size_t i = 0; i < m; ++i)
+            if (const int k = pstate_words(hp.tag[i])) std::memcpy(o->model_data + 24 * i, pstate + 3 * i, 4 * (size_t)k);
     }
     return latched(sc, NXM_OK);
 }

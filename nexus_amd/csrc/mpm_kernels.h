@@ -103,6 +103,18 @@ void launch_set_particles(Globals *g, uint32_t p_in, hipStream_t st);
 // Minimum over each scene's enabled particles of the CFL bound (1e-12 s units), into
 // out[s * stride] by atomicMin (the caller fills it with NONE first).
 void launch_timestep_bound(const WorldDev &w, uint32_t n, uint32_t *out, uint32_t stride, int max_blocks, hipStream_t st);
+// Readback: `comps` consecutive planes from `plane` on, of arena positions [start, start +
+// count), as rows by particle id at out + off.
+struct ReadRows {
+    int plane, comps;
+    size_t off;
+};
+struct ReadList {
+    int n;
+    ReadRows rows[8];
+};
+void launch_read_rows(const Arena &a, uint32_t start, uint32_t count, const ReadList &list, float *out, int cap,
+                      hipStream_t st);
 void launch_canonical(const WorldDev &w, const Arena &prev, uint32_t *pcell, uint32_t *buckets, uint32_t p_hint,
                       hipStream_t st);
 

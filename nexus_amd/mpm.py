@@ -374,7 +374,7 @@ class MpmState:
         """WgPrepReadback: per particle (id order) render colour (n, 4), deformation (n, 4, 4)
         column-major, and position (n, 3)."""
         n = len(self)
-        out = np.zeros((max(n, 1), 24), np.float32)
+        out = np.empty((max(n, 1), 24), np.float32)
         pal = None if group_colors is None else np.ascontiguousarray(group_colors, np.float32).reshape(-1, 4)
         _check(self.lib.nxm_scene_prep_readback(self.handle, int(mode), _ptr(pal) if pal is not None else None,
                                                 0 if pal is None else pal.shape[0], _ptr(out), n))
@@ -506,19 +506,19 @@ class MpmState:
 
     def read_positions(self) -> np.ndarray:
         n = len(self)
-        out = np.zeros((n, 3), np.float32)
+        out = np.empty((n, 3), np.float32)
         _check(self.lib.nxm_scene_read_positions(self.handle, _ptr(out), n))
         return out
 
     def read_particles(self) -> dict:
         n = len(self)
         out = dict(
-            x=np.zeros((n, 3), np.float32), v=np.zeros((n, 3), np.float32), F=np.zeros((n, 9), np.float32),
-            C=np.zeros((n, 9), np.float32), vol0=np.zeros(n, np.float32), radius=np.zeros(n, np.float32),
-            mass=np.zeros(n, np.float32), damping=np.zeros(n, np.float32), phase=np.zeros(n, np.float32),
-            boundary_friction=np.zeros(n, np.float32), group=np.zeros(n, np.uint32),
-            enabled=np.zeros(n, np.uint32), fixed=np.zeros(n, np.uint32), tag=np.zeros(n, np.uint32),
-            model=np.zeros((n, 24), np.uint32),
+            x=np.empty((n, 3), np.float32), v=np.empty((n, 3), np.float32), F=np.empty((n, 9), np.float32),
+            C=np.empty((n, 9), np.float32), vol0=np.empty(n, np.float32), radius=np.empty(n, np.float32),
+            mass=np.empty(n, np.float32), damping=np.empty(n, np.float32), phase=np.empty(n, np.float32),
+            boundary_friction=np.empty(n, np.float32), group=np.empty(n, np.uint32),
+            enabled=np.empty(n, np.uint32), fixed=np.empty(n, np.uint32), tag=np.empty(n, np.uint32),
+            model=np.empty((n, 24), np.uint32),
         )
         soa = _SoA(position=_ptr(out["x"]), velocity=_ptr(out["v"]), def_grad=_ptr(out["F"]), affine=_ptr(out["C"]),
                    init_volume=_ptr(out["vol0"]), init_radius=_ptr(out["radius"]), mass=_ptr(out["mass"]),
