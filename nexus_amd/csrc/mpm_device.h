@@ -218,13 +218,30 @@ __host__ __device__ inline uint32_t spread3(uint32_t v)
     return v;
 }
 
-// First probe slot of a packed block key: the Morton code of its coordinates (low 10
-// bits of each), so spatially close blocks land in close slots and the dense block ids,
-// which are ranks of occupied slots, follow a Morton order.  Blocks whose codes agree
-// modulo the region size collide and are resolved by linear probing.
-__device__ inline uint32_t hash_key(uint32_t k)
+// Probe sequence of a packed block key in a region of mask + 1 slots.  The blocks of a
+// 8^3 group share a base and lie behind it in Morton order: close blocks get close slots, and
+// the dense block ids, which are ranks of occupied slots, follow a Morton order inside a
+// group.  The groups' bases are hashed (a finalizer of Appleby's MurmurHash3), and a slot
+// that is taken leads on by an odd stride of the group's own, which visits every slot.
+// With the Morton code of the whole coordinates as the slot and linear probing, a scene
+// wider than the region's Morton box met runs of thousands of taken slots: at 47,000 blocks
+// in 131,072 slots the sand column's count kernel took 2.8 ms instead of 13 us and its G2P,
+// which inserts the next blocks, 7.4 ms instead of 0.1.
+struct HashProbe {
+    uint32_t slot, stride;
+};
+__device__ inline HashProbe hash_probe(uint32_t key, uint32_t mask)
 {
-    return spread3(k & 0x7FFu) | (spread3((k >> 11) & 0x3FFu) << 1) | (spread3(k >> 21) << 2);
+    constexpr uint32_t B = 3, LOW = (1u << B) - 1u;
+    const uint32_t x = key & 0x7FFu, y = (key >> 11) & 0x3FFu, z = key >> 21;
+    uint32_t h = (x >> B) | ((y >> B) << 8) | ((z >> B) << 16);
+    h ^= h >> 16;
+    h *= 0x85EBCA6Bu;
+    h ^= h >> 13;
+    h *= 0xC2B2AE35u;
+    h ^= h >> 16;
+    const uint32_t low = spread3(x & LOW) | (spread3(y & LOW) << 1) | (spread3(z & LOW) << 2);
+    return HashProbe{((h << (3 * B)) | low) & mask, (h >> 8) | 1u};
 }
 
 // +1 neighbour offsets in the reference's blocks_associated_to_block order

@@ -72,17 +72,18 @@ __device__ inline void xcd_range(uint32_t n, uint32_t &begin, uint32_t &end)
 }
 
 // ------------------------------------------------------------------------------------
-// Hash regions: open addressing, linear probing, 32-bit packed block keys
+// Hash regions: open addressing, double hashing, 32-bit packed block keys
 // (src_mpm_shaders/grid/grid.rs:447-536).  Values are dense block ids.
 
 __device__ inline bool hash_insert(uint32_t *keys, uint32_t mask, uint32_t key, uint32_t &slot)
 {
-    uint32_t s = hash_key(key) & mask;
+    const HashProbe p = hash_probe(key, mask);
+    uint32_t s = p.slot;
     for (uint32_t probe = 0; probe <= mask; ++probe) {
         uint32_t prev = atomicCAS(keys + s, EMPTY_KEY, key);
         if (prev == EMPTY_KEY) { slot = s; return true; }
         if (prev == key) { slot = s; return false; }
-        s = (s + 1) & mask;
+        s = (s + p.stride) & mask;
     }
     slot = NONE;
     return false;
@@ -90,12 +91,13 @@ __device__ inline bool hash_insert(uint32_t *keys, uint32_t mask, uint32_t key, 
 
 __device__ inline uint32_t hash_find(const uint32_t *keys, const uint32_t *vals, uint32_t mask, uint32_t key)
 {
-    uint32_t s = hash_key(key) & mask;
+    const HashProbe p = hash_probe(key, mask);
+    uint32_t s = p.slot;
     for (uint32_t probe = 0; probe <= mask; ++probe) {
         uint32_t k = keys[s];
         if (k == key) return vals[s];
         if (k == EMPTY_KEY) return NONE;
-        s = (s + 1) & mask;
+        s = (s + p.stride) & mask;
     }
     return NONE;
 }
