@@ -885,12 +885,12 @@ class World {
         if (tune_on_ && !tuning_ && tuned_p_ && (p_in_ > 2 * tuned_p_ || 2 * p_in_ < tuned_p_)) start_tuning();
         const nxm_launch_config cfg = tuning_ ? tune_candidate() : cfg_;
         WorldDev w = view();
-        w.p2g_groups = cfg.p2g_groups;
+        w.p2g_groups = p2g_workgroups(cfg.p2g_groups, p_in_);
         w.p2g_block_cost = cfg.p2g_block_cost;
         LaunchConfig lc{};
         lc.p_hint = p_in_;
         lc.persistent_blocks = (int)cfg.grid_groups;
-        lc.p2g_blocks = (int)cfg.p2g_groups;
+        lc.p2g_blocks = (int)w.p2g_groups;
         lc.side = side_;
         lc.fork = fork_;
         lc.join = join_;
@@ -916,7 +916,9 @@ class World {
             HIP_TRY(hipGetLastError());
         }
         clean_ = false;
-        if (graph_on_ && !evs && !tuning_ && !keys) {
+        lc.order = keys || ++order_age_ >= ORDER_EVERY;
+        if (lc.order) order_age_ = 0;
+        if (graph_on_ && !evs && !tuning_ && !keys && !lc.order) {
             // Replays the substep's launches as one graph; recaptured when the launch
             // shapes or any buffer address change.  The graph holds kernels only.
             const GraphKey k{p_in_, b_total_, h_total_, gen_, cfg.p2g_groups, cfg.p2g_block_cost, cfg.grid_groups};
@@ -1650,7 +1652,7 @@ class World {
     {
         const uint32_t cu = (uint32_t)ctx_->num_cus;
         std::vector<nxm_launch_config> c;
-        if (stage == 0) for (uint32_t k : {128u, 256u, 512u}) c.push_back({cu * k, b.p2g_block_cost, b.grid_groups});
+        if (stage == 0) for (uint32_t k : {32u, 128u, 512u}) c.push_back({cu * k, b.p2g_block_cost, b.grid_groups});
         if (stage == 1) for (uint32_t k : {4u, 16u, 64u}) c.push_back({b.p2g_groups, k, b.grid_groups});
         if (stage == 2) for (uint32_t k : {4u, 8u, 16u, 32u, 64u}) c.push_back({b.p2g_groups, b.p2g_block_cost, cu * k});
         return c;
@@ -1789,6 +1791,7 @@ class World {
     uint32_t profile_every_ = 1, profile_seen_ = 0;
     int cur_ = 0;
     uint32_t p_in_ = 0, p_cap_ = 0, b_total_ = 0, h_total_ = 0;
+    uint32_t order_age_ = 0;           // substeps since the particles were last ordered by cell
     size_t ctr_zeroed_ = 0;
     DevBuf<float> arenas_[2];
     DevBuf<uint32_t> pkey_, pdense_, prank_, perm_, sblock_;
@@ -2674,7 +2677,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     const uint32_t b_total = h_total;
     const uint32_t p_cap = (n + 63u) & ~63u;
     const uint32_t cu = (uint32_t)ctx->num_cus;
-    const uint32_t p2g_groups = cu * 32u;
+    const uint32_t p2g_groups = p2g_workgroups(cu * 32u, n);
     const uint32_t scan_stride = (h_total + SCAN_TILE - 1u) / SCAN_TILE + 2u;
     Carver c;
     const size_t o_arena0 = c.take<float>((size_t)NUM_PLANES * p_cap);
@@ -2755,6 +2758,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     lc.p_hint = n;
     lc.persistent_blocks = (int)(cu * 8u);
     lc.p2g_blocks = (int)p2g_groups;
+    lc.order = true;
     launch_noalloc_setup(w, t, dp, lc.persistent_blocks, st);
     launch_clear(w, lc, st);
     launch_substep(w, lc, st, nullptr, true);

@@ -11,11 +11,11 @@ struct WorldDev {
     Arena in, out;                 // particle arenas: read (previous order), written (sorted order)
     uint32_t *pkey;                // per input slot: packed block key
     uint32_t *pdense;              // per input slot: dense block id
-    uint32_t *prank;               // per input slot: rank inside its block
+    uint32_t *prank;               // per input slot: its bound codes, then (counted) its rank inside its block
     uint32_t *perm;                // per sorted position: input slot
     uint32_t *sblock;              // per sorted position: dense block id
     uint32_t *bscene;              // per block: scene slot (NONE = unused id)
-    int4 *bvid;                    // per block: virtual block coordinates
+    int4 *bvid;                    // per block: virtual block coordinates; w: momentum bound code
     uint32_t *bnp;                 // per block: primary particles
     uint32_t *bfirst;              // per block: first sorted position
     uint32_t *bup;                 // per block: 8 ids of vid + {0,1}^3 (reference order)
@@ -24,7 +24,7 @@ struct WorldDev {
     float4 *gridv;                 // per node: velocity after the grid update, mass in w
     uint32_t *hkeys, *hvals;       // hash regions; hvals: dense block id of each occupied slot
     uint32_t *hmark;               // per hash slot: 1 if a particle's primary block
-    uint32_t *bprim;               // per block: 1 if primary (holds particles)
+    uint32_t *bprim;               // per block: nonzero if primary (holds particles); its mass bound code
     uint32_t *bmask;               // per block: colliders that can reach its nodes
     const uint32_t *region_start;  // per active scene, ascending: first hash slot of its region
     const uint32_t *region_scene;  // per active scene: scene slot
@@ -79,12 +79,27 @@ struct WorldDev {
 struct LaunchConfig {
     uint64_t p_hint;               // upper bound of particles (grid sizing only)
     int persistent_blocks;         // cap on workgroups of grid-stride kernels
-    int p2g_blocks;                // workgroups of the per-block kernels
+    int p2g_blocks;                // workgroups of the P2G kernel (p2g_workgroups)
+    bool order = false;            // also order the particles inside their blocks by cell (k_cell_order)
     // CPIC worlds: a second stream (default priority) on which the contact particles' G2P
     // runs beside the plain particles' one, forked and joined with these two events.
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
 };
+
+// Substeps between two orderings of the particles inside their blocks (LaunchConfig::order).
+constexpr uint32_t ORDER_EVERY = 16;
+
+// Waves of a P2G workgroup, and the workgroups launched for p particles when p2g_groups
+// one-wave groups are asked for: a block with particles holds 4 or more in most scenes, so
+// more waves than p / 4 find no block (1000 particles: P2G 14 -> 5 us with 256 instead of
+// 8192).  Whole XCD rounds.
+constexpr int P2G_WAVES = 4;
+inline uint32_t p2g_workgroups(uint32_t groups, uint64_t p)
+{
+    const uint64_t waves = groups < p / 4 ? groups : p / 4;
+    return (uint32_t)((waves / P2G_WAVES + 8) / 8 * 8);
+}
 
 // keys: run k_keys_touch first (the hash and counters emptied by launch_clear); without
 // it the substep uses the keys and block insertions of the previous substep's G2P.

@@ -145,13 +145,58 @@ __global__ void k_clear(WorldDev w)
     }
 }
 
+// One particle's P2G inputs.
+struct P2GIn {
+    float px, py, pz, m;
+    f3 v;
+    m3 C;
+};
+
+__device__ inline P2GIn p2g_load(const WorldDev &w, uint32_t slot)
+{
+    P2GIn p;
+    p.px = w.in.plane(PX)[slot]; p.py = w.in.plane(PY)[slot]; p.pz = w.in.plane(PZ)[slot];
+    p.m = w.in.plane(PMASS)[slot];
+    p.v = mk3(w.in.plane(PVX)[slot], w.in.plane(PVY)[slot], w.in.plane(PVZ)[slot]);
+    p.C.c0 = mk3(w.in.plane(PC0)[slot], w.in.plane(PC1)[slot], w.in.plane(PC2)[slot]);
+    p.C.c1 = mk3(w.in.plane(PC3)[slot], w.in.plane(PC4)[slot], w.in.plane(PC5)[slot]);
+    p.C.c2 = mk3(w.in.plane(PC6)[slot], w.in.plane(PC7)[slot], w.in.plane(PC8)[slot]);
+    return p;
+}
+
+// Bounds of a particle's P2G contributions, |m v + C dpt| (|dpt_j| <= 1.5 h) and m, as the
+// exponents of the powers of two above them: the low half and the high half of one word, 0
+// for none, CODE_HUGE for a bound that is not finite (NaN components are left out, as fmaxf
+// does).  Made where a particle's key is made, from the state still in registers; the
+// count kernel takes a block's maxima, so that P2G reads a block's particles once.
+constexpr int CODE_BIAS = 200;
+constexpr uint32_t CODE_HUGE = 511u;
+__device__ inline uint32_t bound_code(float b)
+{
+    if (!(b > 0.0f)) return 0u;
+    if (!isfinite(b)) return CODE_HUGE;
+    int e;
+    (void)frexpf(b, &e);   // b = m 2^e, m in [0.5, 1): b < 2^e
+    return (uint32_t)(e + CODE_BIAS);
+}
+__device__ inline uint32_t bound_codes(f3 v, const m3 &C, float m, float h)
+{
+    const float cmax = fmaxf(fmaxf(fabsf(C.c0.x), fmaxf(fabsf(C.c0.y), fabsf(C.c0.z))),
+                             fmaxf(fmaxf(fabsf(C.c1.x), fmaxf(fabsf(C.c1.y), fabsf(C.c1.z))),
+                                   fmaxf(fabsf(C.c2.x), fmaxf(fabsf(C.c2.y), fabsf(C.c2.z)))));
+    const float vmax = fmaxf(fabsf(v.x), fmaxf(fabsf(v.y), fabsf(v.z)));
+    const float am = fabsf(m);
+    return bound_code(__builtin_fmaf(4.5f * h, cmax, am * vmax)) | (bound_code(am) << 16);
+}
+
 // Block key of particle slot i at position (x, y, z) of active scene s (written to
-// pkey[i]), and the wave's block insertions: adjacent lanes with the same (scene, key)
+// pkey[i]) and its bound codes (to prank[i]), and the wave's block insertions: adjacent lanes with the same (scene, key)
 // form a run; each run inserts its block (marked primary) and the block's 7 +1
 // neighbours (the active set is P + {0,1}^3, src_mpm/grid/grid.rs:193-200).  Called by
 // every lane of a wave together (invalid lanes with valid = false), so that the lanes'
 // neighbours in the wave are the particles' neighbours in the arena.
-__device__ inline void touch_keys(const WorldDev &w, uint32_t i, bool valid, uint32_t s, float x, float y, float z)
+__device__ inline void touch_keys(const WorldDev &w, uint32_t i, bool valid, uint32_t s, float x, float y, float z,
+                                  uint32_t codes)
 {
     const uint32_t l = lane_id();
     uint32_t key = EMPTY_KEY;
@@ -169,6 +214,7 @@ __device__ inline void touch_keys(const WorldDev &w, uint32_t i, bool valid, uin
             atomicOr(&w.ctr[s].err, ERR_DOMAIN);
         }
         w.pkey[i] = key;
+        w.prank[i] = codes;
     }
     const uint32_t pk = __shfl_up(key, 1, WAVE);
     const uint32_t ps = __shfl_up(s, 1, WAVE);
@@ -226,14 +272,20 @@ __global__ void k_keys_touch(WorldDev w)
         bool valid = i < n;
         uint32_t s = 0;
         float x = 0.0f, y = 0.0f, z = 0.0f;
+        uint32_t codes = 0u;
         if (valid) {
-            s = flags_scene(FL[i]);
+            const uint32_t fl = FL[i];
+            s = flags_scene(fl);
             valid = w.scenes[s].active != 0u;
             x = X[i];
             y = Y[i];
             z = Z[i];
+            if (valid && (fl & FLAG_ENABLED)) {
+                const P2GIn p = p2g_load(w, i);
+                codes = bound_codes(p.v, p.C, p.m, w.scenes[s].h);
+            }
         }
-        touch_keys(w, i, valid, s, x, y, z);
+        touch_keys(w, i, valid, s, x, y, z, codes);
     }
 }
 
@@ -312,6 +364,8 @@ __device__ inline void scan_out(const WorldDev &w, uint32_t i, uint32_t r, uint3
         if (r < w.b_total) {
             w.bscene[r] = s;
             w.bvid[r] = key == OVERFLOW_KEY ? make_int4(OVERFLOW_VID, 0, 0, 0) : unpack_vid(key);
+            // vid.w and bprim take the block's bound codes while its particles are counted
+            // (bprim stays nonzero for a primary block).
             w.bprim[r] = w.hmark[i];
             // This substep's count starts at zero (k_block_count adds to it; the previous
             // substep's stay readable until here; only the dense ids handed out are read).
@@ -511,16 +565,20 @@ __device__ inline void count_part(const WorldDev &w)
     const uint32_t *FL = w.in.uplane(PFLAGS);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nr; i += gridDim.x * blockDim.x) {
         bool valid = i < n;
-        uint32_t d = NONE;
+        uint32_t d = NONE, codes = 0u;
         if (valid) {
             uint32_t s = flags_scene(FL[i]);
             const SceneDev sc = w.scenes[s];
             valid = sc.active != 0u;
             if (valid) {
                 uint32_t key = w.pkey[i];
+                codes = w.prank[i];
                 d = key == OVERFLOW_KEY ? NONE
                                         : hash_find(w.hkeys + sc.h_base, w.hvals + sc.h_base, sc.h_cap - 1u, key);
-                if (d == NONE) d = w.hvals[sc.h_base + sc.h_cap];
+                if (d == NONE) {
+                    d = w.hvals[sc.h_base + sc.h_cap];   // the overflow block: P2G does not take it
+                    codes = 0u;
+                }
                 w.pdense[i] = d;
             }
         }
@@ -530,7 +588,19 @@ __device__ inline void count_part(const WorldDev &w)
         uint64_t heads = __ballot(head);
         uint32_t h = run_head(heads, l);
         uint32_t base = 0;
-        if (head && valid) base = atomicAdd(&w.bnp[d], run_end(heads, l) - l);
+        const uint32_t end = run_end(heads, h);
+        // The run's maxima of the two code halves, at its head.
+        for (uint32_t o = 1; o < WAVE; o <<= 1) {
+            const uint32_t u = __shfl_down(codes, o, WAVE);
+            if (l + o < end) codes = max(codes & 0xFFFFu, u & 0xFFFFu) | (max(codes >> 16, u >> 16) << 16);
+        }
+        if (head && valid) {
+            base = atomicAdd(&w.bnp[d], end - l);
+            if (codes) {
+                atomicMax((uint32_t *)&w.bvid[d].w, codes & 0xFFFFu);
+                atomicMax(&w.bprim[d], codes >> 16);
+            }
+        }
         base = __shfl(base, (int)h, WAVE);
         if (valid) w.prank[i] = base + (l - h);
     }
@@ -555,15 +625,20 @@ __device__ inline void p2g_split(const WorldDev &w)
     if (nb == 0u || G == 0u) return;
     const uint64_t K = w.p2g_block_cost;
     const uint64_t T = (uint64_t)w.g->p_out + K * nb;
-    for (uint32_t d = blockIdx.x * blockDim.x + threadIdx.x; d < nb; d += gridDim.x * blockDim.x) {
-        const uint64_t a = ((uint64_t)w.bfirst[d] + K * d) * G;
-        const uint64_t g_hi = a / T;                                  // last g with start d
-        uint64_t g_lo = 0;                                            // first g with start d
-        if (d > 0) g_lo = (((uint64_t)w.bfirst[d - 1] + K * (d - 1)) * G) / T + 1;
-        for (uint64_t g = g_lo; g <= g_hi && g < G; ++g) w.p2g_start[g] = d;
-        if (d == nb - 1)
-            for (uint64_t g = g_hi + 1; g <= G; ++g) w.p2g_start[g] = nb;
+    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x, gsz = gridDim.x * blockDim.x;
+    // 16 threads share a block's groups where there are several groups per block (few
+    // blocks, or crowded ones: one thread wrote up to hundreds of starts, 51 us for 1000
+    // particles); a thread per block otherwise, since each repeats the two divisions.
+    const uint32_t J = G >= 4u * nb ? 16u : 1u;
+    for (uint64_t t = gid; t < (uint64_t)nb * J; t += gsz) {
+        const uint32_t d = (uint32_t)(t / J);
+        const uint64_t g_hi = ((uint64_t)w.bfirst[d] + K * d) * G / T;   // last g with start d
+        uint64_t g = 0;                                                  // first g with start d
+        if (d > 0) g = (((uint64_t)w.bfirst[d - 1] + K * (d - 1)) * G) / T + 1;
+        for (g += t % J; g <= g_hi && g < G; g += J) w.p2g_start[g] = d;
     }
+    const uint64_t last = ((uint64_t)w.bfirst[nb - 1] + K * (nb - 1)) * G / T;
+    for (uint64_t g = last + 1 + gid; g <= G; g += gsz) w.p2g_start[g] = nb;
 }
 
 __global__ void k_scatter(WorldDev w)
@@ -581,51 +656,109 @@ __global__ void k_scatter(WorldDev w)
     p2g_split(w);
 }
 
+// Order of the particles inside their blocks: by (rank among the particles of their cell,
+// cell), in windows of ORDER_WINDOW.  A wave of P2G then holds particles of different
+// cells, whose stencils meet different nodes at the same instruction: its LDS adds take 9
+// cycles each against 17 in arrival order (8.4 without any conflict; 64 lanes on the 6^3
+// tile).  No result depends on the order.  The output arena keeps it and the sort keeps
+// the arrival order of a block's particles, so it lasts: the pass runs when the host has
+// changed the arena and then once in ORDER_EVERY substeps (particles move about a
+// hundredth of a cell per substep).  One wave per block.
+constexpr int ORDER_PER = 8, ORDER_WINDOW = ORDER_PER * WAVE;
+__global__ void __launch_bounds__(WAVE) k_cell_order(WorldDev w)
+{
+    __shared__ uint32_t count[NODES_PER_BLOCK], before[ORDER_WINDOW];
+    __shared__ uint64_t cells[ORDER_WINDOW];
+    const uint32_t l = threadIdx.x, nb = w.g->n_blocks;
+    for (uint32_t d = blockIdx.x; d < nb; d += gridDim.x) {
+        const int4 v = w.bvid[d];
+        const uint32_t np = w.bnp[d];
+        if (np < 4u || v.x == OVERFLOW_VID) continue;
+        const SceneDev sc = w.scenes[w.bscene[d]];
+        for (uint32_t c0 = 0; c0 < np; c0 += ORDER_WINDOW) {
+            const uint32_t first = w.bfirst[d] + c0, n = min(np - c0, (uint32_t)ORDER_WINDOW);
+            count[l] = 0u;
+            __syncthreads();
+            uint32_t slot[ORDER_PER], cell[ORDER_PER], rank[ORDER_PER];
+            #pragma unroll
+            for (int k = 0; k < ORDER_PER; ++k) slot[k] = k * WAVE + l < n ? w.perm[first + k * WAVE + l] : NONE;
+            #pragma unroll
+            for (int k = 0; k < ORDER_PER; ++k) {
+                if (slot[k] == NONE) continue;
+                const float x = w.in.plane(PX)[slot[k]], y = w.in.plane(PY)[slot[k]], z = w.in.plane(PZ)[slot[k]];
+                // base cell in the block, 0..3 on each axis (a position without one: any cell)
+                const int cx = (int)round_div(x, sc.h, sc.inv_h) - 1 - 4 * v.x;
+                const int cy = (int)round_div(y, sc.h, sc.inv_h) - 1 - 4 * v.y;
+                const int cz = (int)round_div(z, sc.h, sc.inv_h) - 1 - 4 * v.z;
+                cell[k] = (uint32_t)(cx & 3) + 4u * (uint32_t)(cy & 3) + 16u * (uint32_t)(cz & 3);
+                rank[k] = atomicAdd(&count[cell[k]], 1u);
+            }
+            __syncthreads();
+            // cells[r]: the cells with more than r particles; before[r]: particles of rank < r.
+            const uint32_t mine = count[l];
+            uint32_t sum = 0u;
+            for (uint32_t r = 0; sum < n; ++r) {
+                const uint64_t m = __ballot(mine > r);
+                if (l == 0) {
+                    cells[r] = m;
+                    before[r] = sum;
+                }
+                sum += (uint32_t)__popcll(m);
+            }
+            __syncthreads();
+            #pragma unroll
+            for (int k = 0; k < ORDER_PER; ++k)
+                if (slot[k] != NONE)
+                    w.perm[first + before[rank[k]] + (uint32_t)__popcll(cells[rank[k]] & ((1ull << cell[k]) - 1ull))] = slot[k];
+            __syncthreads();
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------
-// P2G: one wave per block.  Each particle adds its 27-node quadratic-B-spline stencil
-// (momentum m v + C dpt and mass, weighted) into a 6^3 LDS tile covering the block and
-// its +1 halo; the tile is then written to the block's staging slot.  Same per-pair
-// arithmetic as gpu_p2g_generic (p2g.rs:240-311): dpt = node - x, contribution
-// (C dpt + m v) w and m w.
+// P2G: one wave per block, or a team of four waves per crowded block.  Each particle adds
+// its 27-node quadratic-B-spline stencil (momentum m v + C dpt and mass, weighted) into a
+// 6^3 LDS tile covering the block and its +1 halo; the tile is then written to the block's
+// staging slot.  Same per-pair arithmetic as gpu_p2g_generic (p2g.rs:240-311): dpt = node -
+// x, contribution (C dpt + m v) w and m w.
 //
 // The tile accumulates in 64-bit fixed point with integer LDS atomics (ds_add_u64):
 // float LDS atomics serialize on gfx950 (~200 cycles per wave-op against ~8 for the
-// 64-bit integer add).  A first pass bounds the block's contributions by 2^e; a tile
-// node receives at most np of them (one per particle of the block), so the scale
-// 2^(62 - e - ceil(log2 np)) keeps every node sum below 2^62 while resolving
-// contributions down to 2^-62 np of the largest.  Integer sums do not depend on the
-// order of the adds, so the tile is bit-reproducible whatever the particle order.
+// 64-bit integer add).  A first pass bounds the block's contributions by 2^e; the scale
+// 2^(51 - e) then resolves each contribution to 2^-52 of that bound, and a node's sum stays
+// below 2^62 for up to 2048 particles in the block (above, the scale gives up a bit per
+// doubling).  Integer sums do not depend on the order of the adds, so the tile is
+// bit-reproducible whatever the particle order.
 
 // 64-bit fixed-point accumulator words of the P2G tile.
 struct Fixed {
     using word = unsigned long long;
-    static constexpr int BITS = 62;
-    // r = v * scale as a two's-complement 64-bit integer hi 2^32 + lo, for |r| < 2^63:
-    // hi = floor(r / 2^32) is exact; lo = r - hi 2^32 lies in [0, 2^32) and is rounded to
-    // float and truncated to an integer.  It is exact when hi >= 0 and |r| >= 2^24 or when
-    // r is a non-negative integer below 2^24; otherwise (a fractional part, or hi = -1 with
-    // lo close to 2^32) it is off by less than 2^8 units, against 2^62 / np units for the
-    // block's largest contribution.  The result depends only on v and the scale,
-    // so integer sums stay independent of the order of the adds.  Non-finite inputs give
-    // garbage that the caller's non-finite mask overrides.
-    __device__ static word to(float v, float scale)
+    // Contributions are formed in double and rounded to the tile's unit by adding 1.5 2^52:
+    // for |a w| < 2^51 the sum's mantissa holds round(a w) in two's complement, and its bit
+    // pattern minus that of 1.5 2^52 (whose low word is zero) is the integer: one fused
+    // multiply-add and one 32-bit subtraction per contribution.  Doubles run at the rate of
+    // floats here, so this replaced the multiply and five operations that split a float into
+    // two 32-bit halves.  The product is exact before that one rounding, so an integer
+    // depends on a and w alone.
+    static constexpr int BITS = 51;
+    static constexpr int FREE_LOG2 = 11;        // particles whose sum needs no headroom bits
+    static constexpr double LIMIT = 0x1p51;     // |a w| below this: an exact conversion
+    __device__ static word of(double a, double w)
     {
-        const float r = v * scale;
-        const float hi = floorf(r * 0x1p-32f);
-        const float lo = __builtin_fmaf(hi, -0x1p32f, r);
-        const uint32_t uhi = (uint32_t)(int32_t)hi;
-        const uint32_t ulo = (uint32_t)lo;
-        return ((unsigned long long)uhi << 32) | ulo;
+        const unsigned long long t = (unsigned long long)__double_as_longlong(__builtin_fma(a, w, 0x1.8p52));
+        return ((unsigned long long)((uint32_t)(t >> 32) - 0x43380000u) << 32) | (uint32_t)t;
     }
     // scale is a power of two: multiplying by its reciprocal is exact
     __device__ static float back(word x, double inv_scale) { return (float)((double)(long long)x * inv_scale); }
 };
 
-__device__ inline float fixed_scale(int bits, int e, uint32_t np)
+// The scale of a block whose contributions are bounded by 2^e, from the bound's code
+// (bound_code).
+__device__ inline float fixed_scale(uint32_t code, uint32_t np)
 {
-    int lg = 0;
-    while ((1u << lg) < np && lg < 31) ++lg;
-    int k = bits - e - lg;
+    const int e = code < 2u || code >= CODE_HUGE ? 0 : (int)code - CODE_BIAS;
+    const int lg = np > 1u ? 32 - __clz((int)(np - 1u)) : 0;   // ceil(log2 np)
+    int k = Fixed::BITS - e - max(lg - Fixed::FREE_LOG2, 0);
     k = k > 126 ? 126 : (k < -126 ? -126 : k);
     return ldexpf(1.0f, k);
 }
@@ -634,112 +767,106 @@ __device__ inline float fixed_scale(int bits, int e, uint32_t np)
 // reference's blocks_associated_to_block order): sizes 64, 32, 32, 16, 32, 16, 16, 8.
 __device__ __constant__ const int REGION_OFFSET[8] = {0, 64, 96, 128, 144, 176, 192, 208};
 
-__device__ inline int bound_exponent(float b)
-{
-    if (!(b > 0.0f) || !isfinite(b)) return 0;
-    int e;
-    frexpf(b, &e);   // b = m 2^e, m in [0.5, 1): b < 2^e
-    return e;
-}
-
-
-__device__ inline float wave_max(float v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-    return v;
-}
-
-// Scatter of one particle's 27 contributions into the block's fixed-point tile.  Lanes
-// start the stencil at different z slabs (lane mod 3): particles of one cell in one wave
-// then add to different nodes at the same instruction instead of serializing on one LDS
-// address; the integer sums do not depend on the order.  CHECK adds the non-finite mask
-// (only for suspect particles, so the common path carries none of the tests).
 // Words of the non-finite mask (one bit per tile word); the word after them flags any.
-// With CPIC the tile holds a second (incompatible) momentum and mass after the first.
 // The tile holds 4 fixed-point fields per node (momentum, mass).  CPIC blocks with
 // particles that carry affinity bits fill it twice: the compatible contributions, flushed
 // to the staging tiles, then the incompatible ones, flushed to the second staging tiles.
-template <bool CPIC> constexpr int tile_fields() { return 4; }
-template <bool CPIC> constexpr int bad_any() { return (tile_fields<CPIC>() * TILE_NODES + 31) / 32; }
+constexpr int TILE_FIELDS = 4;
+constexpr int BAD_ANY = (TILE_FIELDS * TILE_NODES + 31) / 32;
 
 // Which contributions a scatter pass adds: all (no affinity in the block), the compatible
 // ones, or the incompatible ones.
 constexpr int PART_ALL = 0, PART_COMPATIBLE = 1, PART_INCOMPATIBLE = 2;
 
-// K lanes share one particle: K = 1 scatters all 27 stencil nodes, starting at z slab
-// sel (the lane's rotation, so that particles of one cell in one wave add to different
-// nodes at the same instruction); K = 3 the 9 nodes of z slab sel; K = 9 the 3 nodes of
-// row (sz, sy) = (sel / 3, sel % 3); K = 27 node (sel / 9, sel / 3 % 3, sel % 3).  Every
-// node's contribution is computed by the same operations whatever K is.
-template <bool CHECK, bool CPIC, int PART, int K>
-__device__ __forceinline__ void p2g_scatter(unsigned long long *tile, uint32_t *bad, int bx, int by, int bz, int sel,
-                                            const f3 base, const f3 hx, const f3 hy, const f3 hz, const float (&wx)[3],
-                                            const float (&wy)[3], const float (&wz)[3], float smom, float msm,
-                                            const uint32_t *naff, uint32_t pa)
+struct d3 { double x, y, z; };
+__device__ inline d3 scaled(f3 a, double s) { return d3{a.x * s, a.y * s, a.z * s}; }   // exact for 29-bit s
+__device__ inline d3 step(d3 a, d3 h, double s)
+{
+    return d3{__builtin_fma(h.x, s, a.x), __builtin_fma(h.y, s, a.y), __builtin_fma(h.z, s, a.z)};
+}
+__device__ inline float pick(const float (&w)[3], int s) { return s == 0 ? w[0] : (s == 1 ? w[1] : w[2]); }
+
+// One particle's stencil: C dpt + m v at node (sx, sy, sz) is base + sx hx + sy hy + sz hz
+// (three fused steps per node instead of a matrix product), all in double with the block's
+// scales folded in; the weights; the tile index of its base node.
+struct Stencil {
+    d3 base, hx, hy, hz;
+    double mass;
+    float wx[3], wy[3], wz[3];
+    int t0;
+};
+
+// CPIC (p2g.rs:268-302): a particle not compatible with the node adds to the node's
+// incompatible fields (the second pass of the block).
+template <int PART>
+__device__ __forceinline__ bool adds_to(const uint32_t *naff, int t, uint32_t pa)
+{
+    if (PART == PART_ALL) return true;
+    const bool incomp = (pa & 0xFFFFu) != 0u && !aff_compatible(pa, naff[t]);
+    return incomp == (PART == PART_INCOMPATIBLE);
+}
+
+__device__ __forceinline__ void add_node(unsigned long long *tile, int t, d3 a, double mass, double wgt)
+{
+    atomicAdd(&tile[t], Fixed::of(a.x, wgt));
+    atomicAdd(&tile[TILE_NODES + t], Fixed::of(a.y, wgt));
+    atomicAdd(&tile[2 * TILE_NODES + t], Fixed::of(a.z, wgt));
+    atomicAdd(&tile[3 * TILE_NODES + t], Fixed::of(mass, wgt));
+}
+
+// K lanes share one particle: K = 1 scatters all 27 stencil nodes; K = 3 the 9 nodes of z
+// slab sel; K = 9 the 3 nodes of row (sz, sy) = (sel / 3, sel % 3); K = 27 node (sel / 9,
+// sel / 3 % 3, sel % 3).  Every node's contribution is computed by the same operations
+// whatever K is (each step an explicit fused multiply-add, exact for an offset of 0), so
+// which lanes take a particle changes no bit.
+template <int PART, int K>
+__device__ __forceinline__ void p2g_scatter(unsigned long long *tile, const Stencil &q, int sel, const uint32_t *naff,
+                                            uint32_t pa)
 {
     constexpr int NZ = K == 1 ? 3 : 1, NY = K <= 3 ? 3 : 1, NX = K <= 9 ? 3 : 1;
-    #pragma unroll
+    // The z slabs in a loop of nine nodes each: the code of all 27 is several times what the
+    // instruction cache fetches in the time of a small launch.
+    #pragma unroll 1
     for (int kz = 0; kz < NZ; ++kz) {
-        int sz;
-        if (K == 1) sz = kz + sel >= 3 ? kz + sel - 3 : kz + sel;
-        else if (K == 3) sz = sel;
-        else if (K == 9) sz = sel / 3;
-        else sz = sel / 9;
-        // base + sz hz, exactly as base + hz or base + 2 hz (sz hz is exact).
-        const float fsz = (float)sz;
-        const f3 az = mk3(__builtin_fmaf(hz.x, fsz, base.x), __builtin_fmaf(hz.y, fsz, base.y),
-                          __builtin_fmaf(hz.z, fsz, base.z));
-        float wzs = wz[0];
-        wzs = sz == 1 ? wz[1] : wzs;
-        wzs = sz == 2 ? wz[2] : wzs;
+        const int sz = K == 1 ? kz : (K == 3 ? sel : (K == 9 ? sel / 3 : sel / 9));
+        const d3 az = step(q.base, q.hz, (double)sz);
+        const double wzs = (double)pick(q.wz, sz);
         #pragma unroll
         for (int ky = 0; ky < NY; ++ky) {
             const int sy = NY == 3 ? ky : (K == 9 ? sel % 3 : (sel / 3) % 3);
-            f3 ay;
-            float wys;
-            if (NY == 3) {
-                ay = sy == 0 ? az : (sy == 1 ? az + hy : az + hy * 2.0f);
-                wys = wy[sy];
-            } else {
-                const f3 a1 = az + hy, a2 = az + hy * 2.0f;
-                ay = sy == 0 ? az : (sy == 1 ? a1 : a2);
-                wys = sy == 0 ? wy[0] : (sy == 1 ? wy[1] : wy[2]);
-            }
+            const d3 ay = step(az, q.hy, (double)sy);
+            const double wyz = (double)pick(q.wy, sy) * wzs;
             #pragma unroll
             for (int kx = 0; kx < NX; ++kx) {
                 const int sx = NX == 3 ? kx : sel % 3;
-                f3 a;
-                float wxs;
-                if (NX == 3) {
-                    a = sx == 0 ? ay : (sx == 1 ? ay + hx : ay + hx * 2.0f);
-                    wxs = wx[sx];
-                } else {
-                    const f3 a1 = ay + hx, a2 = ay + hx * 2.0f;
-                    a = sx == 0 ? ay : (sx == 1 ? a1 : a2);
-                    wxs = sx == 0 ? wx[0] : (sx == 1 ? wx[1] : wx[2]);
-                }
-                const float wgt = (wxs * wys) * wzs;
-                const f3 vc = a * (wgt * smom);
-                const float mw = msm * wgt;
-                const int tn = (bx + sx) + TILE * (by + sy) + TILE * TILE * (bz + sz);
-                // CPIC (p2g.rs:268-302): a particle not compatible with the node adds to
-                // the node's incompatible fields (the second pass of the block).
-                if (PART != PART_ALL) {
-                    const bool incomp = (pa & 0xFFFFu) != 0u && !aff_compatible(pa, naff[tn]);
-                    if (incomp != (PART == PART_INCOMPATIBLE)) continue;
-                }
-                const int t = tn;
-                atomicAdd(&tile[t], Fixed::to(vc.x, 1.0f));
-                atomicAdd(&tile[TILE_NODES + t], Fixed::to(vc.y, 1.0f));
-                atomicAdd(&tile[2 * TILE_NODES + t], Fixed::to(vc.z, 1.0f));
-                atomicAdd(&tile[3 * TILE_NODES + t], Fixed::to(mw, 1.0f));
-                if (CHECK && (!isfinite(vc.x) || !isfinite(vc.y) || !isfinite(vc.z) || !isfinite(mw))) {
-                    atomicOr(&bad[bad_any<CPIC>()], 1u);
-                    atomicOr(&bad[t >> 5], 1u << (t & 31));
-                    atomicOr(&bad[(TILE_NODES + t) >> 5], 1u << ((TILE_NODES + t) & 31));
-                    atomicOr(&bad[(2 * TILE_NODES + t) >> 5], 1u << ((2 * TILE_NODES + t) & 31));
-                    atomicOr(&bad[(3 * TILE_NODES + t) >> 5], 1u << ((3 * TILE_NODES + t) & 31));
-                }
+                const int t = q.t0 + sx + TILE * sy + TILE * TILE * sz;
+                if (adds_to<PART>(naff, t, pa)) add_node(tile, t, step(ay, q.hx, (double)sx), q.mass, (double)pick(q.wx, sx) * wyz);
+            }
+        }
+    }
+}
+
+// The same for a particle that may give contributions that are not finite or beyond the
+// conversion's range: those are marked, and the node reads NaN.  Rare, so one loop over
+// nodes [q0, q1) of the stencil.
+template <int PART>
+__device__ __forceinline__ void p2g_scatter_checked(unsigned long long *tile, uint32_t *bad, const Stencil &q, int q0,
+                                                    int q1, const uint32_t *naff, uint32_t pa)
+{
+    #pragma unroll 1
+    for (int n = q0; n < q1; ++n) {
+        const int sz = n / 9, sy = n / 3 % 3, sx = n % 3;
+        const int t = q.t0 + sx + TILE * sy + TILE * TILE * sz;
+        if (!adds_to<PART>(naff, t, pa)) continue;
+        const d3 a = step(step(step(q.base, q.hz, (double)sz), q.hy, (double)sy), q.hx, (double)sx);
+        const double wgt = (double)pick(q.wx, sx) * ((double)pick(q.wy, sy) * (double)pick(q.wz, sz));
+        add_node(tile, t, a, q.mass, wgt);
+        auto off = [&](double v) { return !(fabs(v * wgt) < Fixed::LIMIT); };   // NaN too
+        if (off(a.x) || off(a.y) || off(a.z) || off(q.mass)) {
+            atomicOr(&bad[BAD_ANY], 1u);
+            for (int c = 0; c < TILE_FIELDS; ++c) {
+                const int k = c * TILE_NODES + t;
+                atomicOr(&bad[k >> 5], 1u << (k & 31));
             }
         }
     }
@@ -777,18 +904,33 @@ __device__ inline void load_flush_table(uint16_t *fdst, uint32_t l)
     if (l < 54u) reinterpret_cast<uint64_t *>(fdst)[l] = reinterpret_cast<const uint64_t *>(FLUSH_CODE.c)[l];
 }
 
+// A team: the lanes that share one tile.  One wave (its LDS operations execute in order, so
+// it only keeps the compiler from moving them), or the P2G_WAVES waves of a workgroup.
+template <bool TEAM> constexpr int team_lanes() { return TEAM ? P2G_WAVES * WAVE : WAVE; }
+template <bool TEAM> __device__ __forceinline__ void team_sync()
+{
+    if (TEAM) {
+        __syncthreads();
+    } else {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
 // With zero (a block whose particles do not reach every region), the flush also zeroes the
 // words it reads, which are all the words the pass added to: the tile is then clean for the
 // next pass without a full clear.
+template <bool TEAM>
 __device__ __forceinline__ void p2g_flush(unsigned long long *tile, const uint32_t *bad, float4 *stage,
                                           uint32_t d, float smom, float sm, uint32_t l, uint32_t touched,
                                           const uint16_t *fdst, bool zero)
 {
-    __syncthreads();
+    team_sync<TEAM>();
     const double inv_smom = 1.0 / (double)smom, inv_sm = 1.0 / (double)sm;   // exact: powers of two
-    const bool any_bad = bad[bad_any<false>()] != 0u;
+    const bool any_bad = bad[BAD_ANY] != 0u;
     float4 *st = stage + (size_t)d * TILE_NODES;
-    for (int t = (int)l; t < TILE_NODES; t += WAVE) {
+    for (int t = (int)l; t < TILE_NODES; t += team_lanes<TEAM>()) {
         const uint32_t code = fdst[t];
         if (!((touched >> (code >> 8)) & 1u)) continue;   // no particle's stencil reaches region e
         float v4[4];
@@ -807,47 +949,18 @@ __device__ __forceinline__ void p2g_flush(unsigned long long *tile, const uint32
         }
         st[code & 0xFFu] = make_float4(v4[0], v4[1], v4[2], v4[3]);
     }
-    __syncthreads();
+    team_sync<TEAM>();
 }
 
 // Empties the tile (unless the last flush left it clean) and its non-finite marks for the
 // next scatter pass.  Blocks that reach all 8 regions (dense ones) clear here: one tight
 // loop costs them less than zeroing inside the flush.
+template <bool TEAM>
 __device__ __forceinline__ void p2g_clear(unsigned long long *tile, uint32_t *bad, uint32_t l, bool dirty)
 {
     if (dirty)
-        for (int k = l; k < 4 * TILE_NODES; k += WAVE) tile[k] = 0;
-    if (l <= (uint32_t)bad_any<false>()) bad[l] = 0u;
-}
-
-// One particle's P2G inputs.
-struct P2GIn {
-    float px, py, pz, m;
-    f3 v;
-    m3 C;
-};
-
-__device__ inline P2GIn p2g_load(const WorldDev &w, uint32_t slot)
-{
-    P2GIn p;
-    p.px = w.in.plane(PX)[slot]; p.py = w.in.plane(PY)[slot]; p.pz = w.in.plane(PZ)[slot];
-    p.m = w.in.plane(PMASS)[slot];
-    p.v = mk3(w.in.plane(PVX)[slot], w.in.plane(PVY)[slot], w.in.plane(PVZ)[slot]);
-    p.C.c0 = mk3(w.in.plane(PC0)[slot], w.in.plane(PC1)[slot], w.in.plane(PC2)[slot]);
-    p.C.c1 = mk3(w.in.plane(PC3)[slot], w.in.plane(PC4)[slot], w.in.plane(PC5)[slot]);
-    p.C.c2 = mk3(w.in.plane(PC6)[slot], w.in.plane(PC7)[slot], w.in.plane(PC8)[slot]);
-    return p;
-}
-
-// Bounds of |m v + C dpt| (|dpt_j| <= 1.5 h) and of m for one particle.
-__device__ inline void p2g_bound(const P2GIn &p, float h, float &bmom, float &bm)
-{
-    float cmax = fmaxf(fmaxf(fabsf(p.C.c0.x), fmaxf(fabsf(p.C.c0.y), fabsf(p.C.c0.z))),
-                       fmaxf(fmaxf(fabsf(p.C.c1.x), fmaxf(fabsf(p.C.c1.y), fabsf(p.C.c1.z))),
-                             fmaxf(fabsf(p.C.c2.x), fmaxf(fabsf(p.C.c2.y), fabsf(p.C.c2.z)))));
-    const float vmax = fmaxf(fabsf(p.v.x), fmaxf(fabsf(p.v.y), fabsf(p.v.z)));
-    bmom = fmaxf(bmom, fabsf(p.m) * vmax + 4.5f * h * cmax);
-    bm = fmaxf(bm, fabsf(p.m));
+        for (int k = l; k < TILE_FIELDS * TILE_NODES; k += team_lanes<TEAM>()) tile[k] = 0;
+    if (l <= (uint32_t)BAD_ANY) bad[l] = 0u;
 }
 
 // Staging regions of a block's tile that a particle with base cell (bx, by, bz) in the
@@ -868,115 +981,86 @@ __device__ inline uint32_t spill_mask(int bx, int by, int bz)
     return m;
 }
 
-// Scatter of one enabled particle of block vid into the tile.
-template <bool CPIC, int PART, int K = 1>
-__device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *bad, const P2GIn &p, const int4 v,
-                                        const SceneDev &sc, float smom, float sm, float bmom, float bm, uint32_t sel,
-                                        const uint32_t *naff, uint32_t pa)
+// The quadratic B-spline weights of one axis, f in [0.5, 1.5] cells from the base node.
+__device__ __forceinline__ void stencil_weights(float f, float (&w)[3])
 {
-    const float h = sc.h;
-    const float px = p.px, py = p.py, pz = p.pz, m = p.m;
-    const f3 mom = p.v * m;
-    const m3 &C = p.C;
+    const float a = 1.5f - f, b = f - 1.0f, c = f - 0.5f;
+    w[0] = 0.5f * a * a;
+    w[1] = __builtin_fmaf(-b, b, 0.75f);
+    w[2] = 0.5f * c * c;
+}
+
+// What a wave knows of the block it scatters.
+struct BlockScales {
+    int4 v;
+    float h, ih, smom, sm;
+    bool huge;              // a bound beyond 2^100: check every contribution
+};
+__device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t s, int4 v, uint32_t mass_code, uint32_t np)
+{
+    BlockScales b;
+    b.v = v;
+    b.h = ld_uniform(&w.scenes[s].h);
+    b.ih = ld_uniform(&w.scenes[s].inv_h);
+    b.smom = fixed_scale((uint32_t)v.w, np);
+    b.sm = fixed_scale(mass_code, np);
+    b.huge = (uint32_t)v.w > CODE_BIAS + 100u || mass_code > CODE_BIAS + 100u;
+    return b;
+}
+
+// Scatter of one particle, by this lane as lane sel of the K that share it; returns the
+// staging regions it reaches (0: its base cell is not in the block).
+template <int PART, int K>
+__device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *bad, const P2GIn &p, const BlockScales &b,
+                                            uint32_t sel, const uint32_t *naff, uint32_t pa)
+{
+    const float h = b.h, ih = b.ih;
     // With finite inputs and a finite block bound far below FLT_MAX every contribution is
-    // finite (|contribution| <= bound), so only suspect particles check each contribution
-    // for the non-finite mask.
-    float amax = fmaxf(fabsf(px), fmaxf(fabsf(py), fabsf(pz)));
-    amax = fmaxf(amax, fmaxf(fabsf(mom.x), fmaxf(fabsf(mom.y), fabsf(mom.z))));
-    amax = fmaxf(amax, fabsf(m));
-    #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const f3 col = k == 0 ? C.c0 : (k == 1 ? C.c1 : C.c2);
-        amax = fmaxf(amax, fmaxf(fabsf(col.x), fmaxf(fabsf(col.y), fabsf(col.z))));
-    }
-    // fmaxf drops NaN operands: test them separately.
-    const bool any_nan = px != px || py != py || pz != pz || mom.x != mom.x || mom.y != mom.y ||
-                         mom.z != mom.z || m != m || C.c0.x != C.c0.x || C.c0.y != C.c0.y ||
-                         C.c0.z != C.c0.z || C.c1.x != C.c1.x || C.c1.y != C.c1.y ||
-                         C.c1.z != C.c1.z || C.c2.x != C.c2.x || C.c2.y != C.c2.y || C.c2.z != C.c2.z;
-    const bool suspect = any_nan || !(amax < 0x1p100f) || !(bmom < 0x1p100f) || !(bm < 0x1p100f);
+    // finite (|contribution| <= bound): only other particles take the checked scatter.
+    float z = p.px * 0.0f;   // NaN if any input is not finite
+    z = __builtin_fmaf(p.py, 0.0f, __builtin_fmaf(p.pz, 0.0f, __builtin_fmaf(p.m, 0.0f, z)));
+    z = __builtin_fmaf(p.v.x, 0.0f, __builtin_fmaf(p.v.y, 0.0f, __builtin_fmaf(p.v.z, 0.0f, z)));
+    z = __builtin_fmaf(p.C.c0.x, 0.0f, __builtin_fmaf(p.C.c0.y, 0.0f, __builtin_fmaf(p.C.c0.z, 0.0f, z)));
+    z = __builtin_fmaf(p.C.c1.x, 0.0f, __builtin_fmaf(p.C.c1.y, 0.0f, __builtin_fmaf(p.C.c1.z, 0.0f, z)));
+    z = __builtin_fmaf(p.C.c2.x, 0.0f, __builtin_fmaf(p.C.c2.y, 0.0f, __builtin_fmaf(p.C.c2.z, 0.0f, z)));
     // Base node of the stencil and its offset from the particle.
-    const float ih = sc.inv_h;
-    const float cx = round_div(px, h, ih) - 1.0f, cy = round_div(py, h, ih) - 1.0f, cz = round_div(pz, h, ih) - 1.0f;
-    const int bx = (int)cx - 4 * v.x, by = (int)cy - 4 * v.y, bz = (int)cz - 4 * v.z;
+    const float cx = round_div(p.px, h, ih) - 1.0f, cy = round_div(p.py, h, ih) - 1.0f, cz = round_div(p.pz, h, ih) - 1.0f;
+    const int bx = (int)cx - 4 * b.v.x, by = (int)cy - 4 * b.v.y, bz = (int)cz - 4 * b.v.z;
     // A particle's primary block holds its base cell: bx, by, bz are in [0, 3] for every
     // finite position; anything else contributes nothing.
-    const bool inside = (unsigned)bx < 4u && (unsigned)by < 4u && (unsigned)bz < 4u;
-    const f3 d0 = mk3(cx * h - px, cy * h - py, cz * h - pz);
-    float wx[3], wy[3], wz[3];
-    {
-        const float fx = -d0.x * ih, fy = -d0.y * ih, fz = -d0.z * ih;
-        wx[0] = 0.5f * (1.5f - fx) * (1.5f - fx); wx[1] = 0.75f - (fx - 1.0f) * (fx - 1.0f); wx[2] = 0.5f * (fx - 0.5f) * (fx - 0.5f);
-        wy[0] = 0.5f * (1.5f - fy) * (1.5f - fy); wy[1] = 0.75f - (fy - 1.0f) * (fy - 1.0f); wy[2] = 0.5f * (fy - 0.5f) * (fy - 0.5f);
-        wz[0] = 0.5f * (1.5f - fz) * (1.5f - fz); wz[1] = 0.75f - (fz - 1.0f) * (fz - 1.0f); wz[2] = 0.5f * (fz - 0.5f) * (fz - 0.5f);
-    }
-    // C dpt + m v at node (sx, sy, sz) = (C d0 + m v) + sx (h C.c0) + sy (h C.c1) + sz (h C.c2):
-    // three adds per node instead of a matrix product.  The fixed-point scales are powers of
-    // two, so folding them into the weight changes no bits.
-    const f3 base = mul(C, d0) + mom;
-    const f3 hx = C.c0 * h, hy = C.c1 * h, hz = C.c2 * h;
-    const float msm = m * sm;
-    if (!inside) return 0u;
-    if (suspect)
-        p2g_scatter<true, CPIC, PART, K>(tile, bad, bx, by, bz, (int)sel, base, hx, hy, hz, wx, wy, wz, smom, msm, naff, pa);
-    else
-        p2g_scatter<false, CPIC, PART, K>(tile, bad, bx, by, bz, (int)sel, base, hx, hy, hz, wx, wy, wz, smom, msm, naff, pa);
+    if (!((unsigned)bx < 4u && (unsigned)by < 4u && (unsigned)bz < 4u)) return 0u;
+    // Every operation that could be contracted is an explicit fused one: this function is
+    // inlined once per way of taking a particle, and the copies must agree in every bit.
+    const f3 d0 = mk3(__builtin_fmaf(cx, h, -p.px), __builtin_fmaf(cy, h, -p.py), __builtin_fmaf(cz, h, -p.pz));
+    Stencil q;
+    q.t0 = bx + TILE * by + TILE * TILE * bz;
+    stencil_weights(-d0.x * ih, q.wx);
+    stencil_weights(-d0.y * ih, q.wy);
+    stencil_weights(-d0.z * ih, q.wz);
+    // The scales are powers of two and products of two floats are exact in double.
+    const double ds = (double)b.smom, hs = (double)h * ds;
+    q.base = scaled(p.v, (double)p.m * ds);
+    q.base = step(q.base, scaled(p.C.c0, ds), (double)d0.x);
+    q.base = step(q.base, scaled(p.C.c1, ds), (double)d0.y);
+    q.base = step(q.base, scaled(p.C.c2, ds), (double)d0.z);
+    q.hx = scaled(p.C.c0, hs);
+    q.hy = scaled(p.C.c1, hs);
+    q.hz = scaled(p.C.c2, hs);
+    q.mass = (double)p.m * (double)b.sm;
+    if (b.huge || !(z == 0.0f)) p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K), naff, pa);
+    else p2g_scatter<PART, K>(tile, q, (int)sel, naff, pa);
     return spill_mask(bx, by, bz);
-}
-
-// Scatter of the particle at sorted position pos (when enabled; the incompatible pass
-// takes only particles with affinity bits).
-template <bool CPIC, int PART, int K>
-__device__ __forceinline__ uint32_t p2g_pos(const WorldDev &w, unsigned long long *tile, uint32_t *bad, uint32_t pos,
-                                            const int4 v, const SceneDev &sc, float smom, float sm, float bmom, float bm,
-                                            uint32_t sel, const uint32_t *naff)
-{
-    const uint32_t slot = w.perm[pos];
-    if (!(w.in.uplane(PFLAGS)[slot] & FLAG_ENABLED)) return 0u;
-    const uint32_t pa = PART == PART_ALL ? 0u : w.out.uplane(PAFF)[pos];
-    if (PART == PART_INCOMPATIBLE && (pa & 0xFFFFu) == 0u) return 0u;
-    return p2g_one<CPIC, PART, K>(tile, bad, p2g_load(w, slot), v, sc, smom, sm, bmom, bm, sel, naff, pa);
-}
-
-// One scatter pass over the np particles of a block starting at sorted position first:
-// whole chunks of 64 one particle per lane; the remainder r with K lanes per particle,
-// K = 27, 9, 3 or 1 for r <= 2, 7, 21 or more, so that a small remainder costs a fraction
-// of a full 27-node pass.
-template <bool CPIC, int PART>
-__device__ __forceinline__ uint32_t p2g_block_pass(const WorldDev &w, unsigned long long *tile, uint32_t *bad,
-                                                   uint32_t first, uint32_t np, const int4 v, const SceneDev &sc,
-                                                   float smom, float sm, float bmom, float bm, uint32_t l,
-                                                   const uint32_t *naff)
-{
-    const uint32_t full = np / WAVE * WAVE, rem = np - full;
-    uint32_t spill = 0u;
-    for (uint32_t c = 0; c < full; c += WAVE)
-        spill |= p2g_pos<CPIC, PART, 1>(w, tile, bad, first + c + l, v, sc, smom, sm, bmom, bm, l % 3u, naff);
-    if (rem == 0u) return spill;
-    const uint32_t at = first + full;
-    if (rem <= 2u) {
-        if (l < 27u * rem)
-            spill |= p2g_pos<CPIC, PART, 27>(w, tile, bad, at + l / 27u, v, sc, smom, sm, bmom, bm, l % 27u, naff);
-    } else if (rem <= 7u) {
-        if (l < 9u * rem)
-            spill |= p2g_pos<CPIC, PART, 9>(w, tile, bad, at + l / 9u, v, sc, smom, sm, bmom, bm, l % 9u, naff);
-    } else if (rem <= 21u) {
-        if (l < 3u * rem)
-            spill |= p2g_pos<CPIC, PART, 3>(w, tile, bad, at + l / 3u, v, sc, smom, sm, bmom, bm, l % 3u, naff);
-    } else if (l < rem) {
-        spill |= p2g_pos<CPIC, PART, 1>(w, tile, bad, at + l, v, sc, smom, sm, bmom, bm, l % 3u, naff);
-    }
-    return spill;
 }
 
 // Node affinity words of block d's 6^3 tile (CPIC scenes; zero, compatible with every
 // particle, elsewhere and for missing blocks).
-__device__ inline void load_tile_affinity(const WorldDev &w, uint32_t d, bool cpic, uint32_t *naff, uint32_t l)
+template <bool TEAM>
+__device__ inline void load_tile_affinity(const WorldDev &w, uint32_t d, uint32_t *naff, uint32_t l)
 {
-    for (int t = l; t < TILE_NODES; t += WAVE) {
+    for (int t = l; t < TILE_NODES; t += team_lanes<TEAM>()) {
         const int tx = t % TILE, ty = (t / TILE) % TILE, tz = t / (TILE * TILE);
         const int e = 4 * (tx >> 2) + 2 * (ty >> 2) + (tz >> 2);
-        const uint32_t blk = cpic ? w.bup[8 * (size_t)d + e] : NONE;
+        const uint32_t blk = w.bup[8 * (size_t)d + e];
         naff[t] = blk == NONE ? 0u : w.ncdf[(size_t)blk * NODES_PER_BLOCK + (tx & 3) + 4 * (ty & 3) + 16 * (tz & 3)].y;
     }
 }
@@ -1001,111 +1085,222 @@ __device__ inline void unlink_untouched(const WorldDev &w, uint32_t d, uint32_t 
     }
 }
 
-template <bool CPIC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_p2g(WorldDev w)
+// A particle of the input arena for P2G; off: none, or a disabled one.
+struct P2GLane {
+    P2GIn p;
+    bool on;
+};
+__device__ __forceinline__ P2GLane p2g_fetch(const WorldDev &w, uint32_t slot)
 {
-    using FX = Fixed;
-    constexpr int NF = tile_fields<CPIC>();
-    __shared__ typename FX::word tile[NF * TILE_NODES];
-    __shared__ uint32_t bad[bad_any<CPIC>() + 1];   // non-finite contributions; last word: any at all
-    __shared__ uint32_t naff[CPIC ? TILE_NODES : 1];
-    const uint32_t l = threadIdx.x;
-    const uint32_t *FL = w.in.uplane(PFLAGS);
-    __shared__ __align__(8) uint16_t fdst[TILE_NODES];
-    load_flush_table(fdst, l);   // read after the first __syncthreads
-    bool dirty = true;           // the tile may hold non-zero words (p2g_clear, p2g_flush)
-    // Cost-balanced block range, XCD-contiguous (see p2g_split and xcd_range).
-    const uint32_t G = gridDim.x, b = blockIdx.x;
-    const uint32_t g = (G % NUM_XCD == 0) ? (b % NUM_XCD) * (G / NUM_XCD) + b / NUM_XCD : b;
-    // Per-block words by scalar loads in the plain variant (the CPIC one spills more with them).
-    const uint32_t dbegin = ld_maybe_uniform<!CPIC>(w.p2g_start + g), dend = ld_maybe_uniform<!CPIC>(w.p2g_start + g + 1);
-    for (uint32_t d = dbegin; d < dend; ++d) {
-        const uint32_t s = ld_maybe_uniform<!CPIC>(w.bscene + d);
-        const uint32_t np = ld_maybe_uniform<!CPIC>(w.bnp + d);
-        const int4 v = ld_maybe_uniform<!CPIC>(w.bvid + d);
-        if (np == 0u || v.x == OVERFLOW_VID) continue;
-        const SceneDev sc = w.scenes[s];
-        const float h = sc.h;
-        const uint32_t first = ld_maybe_uniform<!CPIC>(w.bfirst + d);
-        float bmom = 0.0f, bm = 0.0f;
-        if (np <= (uint32_t)WAVE && np > 21u) {
-            // One particle per lane: load it once, bound, then scatter from registers.
-            P2GIn p{};
-            bool on = false;
-            uint32_t pa = 0u, spill = 0u;
-            if (l < np) {
-                const uint32_t slot = w.perm[first + l];
-                on = (FL[slot] & FLAG_ENABLED) != 0u;
-                if (on) {
-                    p = p2g_load(w, slot);
-                    p2g_bound(p, h, bmom, bm);
-                    if (CPIC && w.breach[d]) pa = w.out.uplane(PAFF)[first + l];
-                }
-            }
-            bmom = wave_max(bmom);
-            bm = wave_max(bm);
-            const float smom = fixed_scale(FX::BITS, bound_exponent(bmom), np);
-            const float sm = fixed_scale(FX::BITS, bound_exponent(bm), np);
-            const bool inc = CPIC && __ballot((pa & 0xFFFFu) != 0u) != 0ull;
-            p2g_clear(tile, bad, l, dirty);
-            if (inc) load_tile_affinity(w, d, true, naff, l);
+    P2GLane r{};
+    if (slot != NONE) {
+        r.on = (w.in.uplane(PFLAGS)[slot] & FLAG_ENABLED) != 0u;
+        r.p = p2g_load(w, slot);
+    }
+    return r;
+}
+
+// One turn of a wave on a block: its particles [64 c, 64 c + 64), one per lane; the block's
+// last turn, of r < 64 particles, with K lanes per particle: K = 27, 9, 3 or 1 for r <= 2,
+// 7, 21 or more, so that a small remainder costs a fraction of a full 27-node pass.
+struct Turn {
+    uint32_t d, np, first, c, s, mass_code;   // np = 0: none
+    int4 v;
+};
+__device__ __forceinline__ uint32_t turn_lanes(const Turn &t)
+{
+    const uint32_t r = t.np - WAVE * t.c;
+    return r <= 2u ? 27u : (r <= 7u ? 9u : (r <= 21u ? 3u : 1u));
+}
+__device__ __forceinline__ uint32_t turn_slot(const WorldDev &w, const Turn &t, uint32_t l)
+{
+    if (t.np == 0u) return NONE;
+    const uint32_t k = turn_lanes(t);
+    const uint32_t i = WAVE * t.c + (k == 1u ? l : (k == 3u ? l / 3u : (k == 9u ? l / 9u : l / 27u)));
+    return i < t.np ? w.perm[t.first + i] : NONE;
+}
+
+// Staging regions reached, over a wave or a team.
+template <bool TEAM>
+__device__ __forceinline__ uint32_t team_touched(uint32_t *words, uint32_t l, uint32_t spill)
+{
+    uint32_t m = wave_or_mask8(spill);
+    if (!TEAM) return m;
+    if (l % WAVE == 0) words[l / WAVE] = m;
+    __syncthreads();
+    #pragma unroll
+    for (int k = 0; k < P2G_WAVES; ++k) m |= words[k];
+    return m;
+}
+
+// One block by a team, or (CPIC) by one wave: the crowded blocks, and the CPIC blocks with
+// nodes in reach of a collider.  Each wave takes its turns of 64 particles, the next one's
+// loads under the scatter of this one.
+template <bool CPIC, bool TEAM, int PART>
+__device__ __forceinline__ uint32_t p2g_turns(const WorldDev &w, unsigned long long *tile, uint32_t *bad, const BlockScales &b,
+                                              uint32_t first, uint32_t np, uint32_t l, const uint32_t *naff)
+{
+    uint32_t spill = 0u;
+    auto slot_of = [&](uint32_t i) { return i < np ? w.perm[first + i] : NONE; };
+    auto aff_of = [&](uint32_t i) { return PART != PART_ALL && i < np ? w.out.uplane(PAFF)[first + i] : 0u; };
+    uint32_t next = slot_of(l + team_lanes<TEAM>());
+    P2GLane q = p2g_fetch(w, slot_of(l));
+    for (uint32_t i = l; i - l % WAVE < np; i += team_lanes<TEAM>()) {
+        const uint32_t pa = aff_of(i);
+        const P2GLane now = q;
+        q = p2g_fetch(w, next);
+        next = slot_of(i + 2 * team_lanes<TEAM>());
+        if (now.on && (PART != PART_INCOMPATIBLE || (pa & 0xFFFFu) != 0u))
+            spill |= p2g_one<PART, 1>(tile, bad, now.p, b, 0u, naff, pa);
+    }
+    return spill;
+}
+
+template <bool CPIC, bool TEAM>
+__device__ __forceinline__ void p2g_block(const WorldDev &w, uint32_t d, uint32_t np, const int4 v, uint32_t l,
+                                          unsigned long long *tile, uint32_t *bad, uint32_t *naff, const uint16_t *fdst,
+                                          uint32_t *words, bool &dirty)
+{
+    const uint32_t first = ld_uniform(w.bfirst + d);
+    const BlockScales b = block_scales(w, ld_uniform(w.bscene + d), v, ld_uniform(w.bprim + d), np);
+    bool inc = false;
+    if (CPIC && ld_uniform(w.breach + d)) {
+        for (uint32_t i = l; i < np; i += team_lanes<TEAM>())
+            inc |= (w.out.uplane(PAFF)[first + i] & 0xFFFFu) != 0u && (w.in.uplane(PFLAGS)[w.perm[first + i]] & FLAG_ENABLED);
+        inc = __ballot(inc) != 0ull;
+        if (TEAM) {
+            if (l % WAVE == 0) words[l / WAVE] = inc ? 1u : 0u;
             __syncthreads();
-            if (on) {
-                if (inc) spill = p2g_one<CPIC, PART_COMPATIBLE>(tile, bad, p, v, sc, smom, sm, bmom, bm, l % 3u, naff, pa);
-                else spill = p2g_one<CPIC, PART_ALL>(tile, bad, p, v, sc, smom, sm, bmom, bm, l % 3u, naff, pa);
-            }
-            const uint32_t touched = wave_or_mask8(spill);
-            p2g_flush(tile, bad, reinterpret_cast<float4 *>(w.stage), d, smom, sm, l, touched, fdst, touched != 0xFFu);
-            dirty = touched == 0xFFu;
-            if (CPIC && l == 0) w.binc[d] = inc ? 1u : 0u;
-            if (CPIC && inc) {
-                // Second pass: the incompatible contributions of the particles with affinity.
-                p2g_clear(tile, bad, l, dirty);
-                __syncthreads();
-                if (on && (pa & 0xFFFFu) != 0u)
-                    p2g_one<CPIC, PART_INCOMPATIBLE>(tile, bad, p, v, sc, smom, sm, bmom, bm, l % 3u, naff, pa);
-                p2g_flush(tile, bad, reinterpret_cast<float4 *>(w.stage_i), d, smom, sm, l, touched, fdst, touched != 0xFFu);
-                dirty = touched == 0xFFu;
-            }
-            unlink_untouched(w, d, touched, l);
-            continue;
+            for (int k = 0; k < P2G_WAVES; ++k) inc |= words[k] != 0u;
         }
-        // Pass 1: bounds over the block; pass 2: the scatter (p2g_block_pass).
-        bool anyc = false;
-        for (uint32_t c = 0; c < np; c += WAVE) {
-            const uint32_t pos = first + c + l;
-            if (pos < first + np) {
-                const uint32_t slot = w.perm[pos];
-                if (FL[slot] & FLAG_ENABLED) {
-                    p2g_bound(p2g_load(w, slot), h, bmom, bm);
-                    if (CPIC && w.breach[d]) anyc |= (w.out.uplane(PAFF)[pos] & 0xFFFFu) != 0u;
-                }
-            }
-        }
-        bmom = wave_max(bmom);
-        bm = wave_max(bm);
-        const float smom = fixed_scale(FX::BITS, bound_exponent(bmom), np);
-        const float sm = fixed_scale(FX::BITS, bound_exponent(bm), np);
-        const bool inc = CPIC && __ballot(anyc) != 0ull;
-        p2g_clear(tile, bad, l, dirty);
-        if (inc) load_tile_affinity(w, d, true, naff, l);
-        __syncthreads();
-        const uint32_t spill =
-            inc ? p2g_block_pass<CPIC, PART_COMPATIBLE>(w, tile, bad, first, np, v, sc, smom, sm, bmom, bm, l, naff)
-                : p2g_block_pass<CPIC, PART_ALL>(w, tile, bad, first, np, v, sc, smom, sm, bmom, bm, l, naff);
-        const uint32_t touched = wave_or_mask8(spill);
-        p2g_flush(tile, bad, reinterpret_cast<float4 *>(w.stage), d, smom, sm, l, touched, fdst, touched != 0xFFu);
+    }
+    p2g_clear<TEAM>(tile, bad, l, dirty);
+    if (CPIC && inc) load_tile_affinity<TEAM>(w, d, naff, l);
+    team_sync<TEAM>();
+    uint32_t spill;
+    if (CPIC && inc) spill = p2g_turns<CPIC, TEAM, PART_COMPATIBLE>(w, tile, bad, b, first, np, l, naff);
+    else spill = p2g_turns<CPIC, TEAM, PART_ALL>(w, tile, bad, b, first, np, l, naff);
+    const uint32_t touched = team_touched<TEAM>(words, l, spill);
+    p2g_flush<TEAM>(tile, bad, reinterpret_cast<float4 *>(w.stage), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+    dirty = touched == 0xFFu;
+    if (CPIC && inc) {
+        // Second pass: the incompatible contributions of the particles with affinity.
+        p2g_clear<TEAM>(tile, bad, l, dirty);
+        team_sync<TEAM>();
+        p2g_turns<CPIC, TEAM, PART_INCOMPATIBLE>(w, tile, bad, b, first, np, l, naff);
+        p2g_flush<TEAM>(tile, bad, reinterpret_cast<float4 *>(w.stage_i), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
         dirty = touched == 0xFFu;
-        if (CPIC && l == 0) w.binc[d] = inc ? 1u : 0u;
-        if (CPIC && inc) {
-            // Second pass: the incompatible contributions of the particles with affinity.
-            p2g_clear(tile, bad, l, dirty);
-            __syncthreads();
-            p2g_block_pass<CPIC, PART_INCOMPATIBLE>(w, tile, bad, first, np, v, sc, smom, sm, bmom, bm, l, naff);
-            p2g_flush(tile, bad, reinterpret_cast<float4 *>(w.stage_i), d, smom, sm, l, touched, fdst, touched != 0xFFu);
-            dirty = touched == 0xFFu;
+    }
+    unlink_untouched(w, d, touched, l);
+    if (CPIC && l == 0) w.binc[d] = inc ? 1u : 0u;
+}
+
+// Workgroups of P2G_WAVES waves, each with a cost-balanced range of blocks (p2g_split), the
+// ranges of an XCD contiguous.  The waves take the range's blocks of up to TEAM_MIN
+// particles one by one from a counter, each with a tile of its own; the crowded blocks are
+// then taken by all the waves together on one tile: a block's particles are one serial
+// chain otherwise (a block of 512 took 8 turns of 64, and a body of 32,768 particles at 8
+// per cell kept 64 waves of the chip busy).
+// A wave works ahead: while it scatters one turn, the next turn's particles (of the same
+// block or the next) are being loaded and the slots of the one after are read, so that the
+// chain slot -> particle -> LDS adds of a block is not waited for.
+constexpr uint32_t TEAM_MIN = 128;
+template <bool CPIC>
+__global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(4))) k_p2g(WorldDev w)
+{
+    __shared__ typename Fixed::word tiles[P2G_WAVES][TILE_FIELDS * TILE_NODES];
+    __shared__ uint32_t bads[P2G_WAVES][BAD_ANY + 1];   // non-finite contributions; last word: any at all
+    __shared__ uint32_t naffs[CPIC ? P2G_WAVES : 1][CPIC ? TILE_NODES : 1];
+    __shared__ __align__(8) uint16_t fdst[TILE_NODES];
+    __shared__ uint32_t words[P2G_WAVES], queue[2];
+    const uint32_t G = gridDim.x, bx = blockIdx.x;
+    const uint32_t g = (G % NUM_XCD == 0) ? (bx % NUM_XCD) * (G / NUM_XCD) + bx / NUM_XCD : bx;
+    const uint32_t begin = ld_uniform(w.p2g_start + g), end = ld_uniform(w.p2g_start + g + 1);
+    if (begin == end) return;
+    load_flush_table(fdst, threadIdx.x);
+    if (threadIdx.x < 2u) queue[threadIdx.x] = begin;
+    __syncthreads();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id();
+    unsigned long long *tile = tiles[wave];
+    uint32_t *bad = bads[wave], *naff = naffs[CPIC ? wave : 0];
+    bool dirty = true;
+    // Next block of a queue whose particles are taken by one wave (CPIC: those in reach of
+    // a collider come from the second queue).
+    auto pop = [&](int which, Turn &t) {
+        for (;;) {
+            uint32_t at = 0u;
+            if (l == 0) at = atomicAdd(&queue[which], 1u);
+            t.d = __builtin_amdgcn_readfirstlane(at);
+            t.np = 0u;
+            if (t.d >= end) return;
+            const uint32_t np = ld_uniform(w.bnp + t.d);
+            if (np == 0u || np > TEAM_MIN) continue;
+            t.v = ld_uniform(w.bvid + t.d);
+            if (t.v.x == OVERFLOW_VID) continue;
+            if (CPIC && (ld_uniform(w.breach + t.d) != 0u) != (which == 1)) continue;
+            t.np = np;
+            t.c = 0u;
+            t.first = ld_uniform(w.bfirst + t.d);
+            t.s = ld_uniform(w.bscene + t.d);
+            t.mass_code = ld_uniform(w.bprim + t.d);
+            return;
         }
-        unlink_untouched(w, d, touched, l);
+    };
+    auto advance = [&](const Turn &t) {
+        Turn n = t;
+        if (WAVE * (t.c + 1u) < t.np) ++n.c;
+        else if (t.np) pop(0, n);
+        return n;
+    };
+    Turn t0;
+    pop(0, t0);
+    Turn t1 = advance(t0);
+    P2GLane q = p2g_fetch(w, turn_slot(w, t0, l));
+    uint32_t slot1 = turn_slot(w, t1, l), spill = 0u;
+    while (t0.np) {
+        const Turn t2 = advance(t1);
+        const uint32_t slot2 = turn_slot(w, t2, l);
+        const P2GLane q1 = p2g_fetch(w, slot1);
+        const BlockScales b = block_scales(w, t0.s, t0.v, t0.mass_code, t0.np);
+        if (t0.c == 0u) {
+            p2g_clear<false>(tile, bad, l, dirty);
+            team_sync<false>();
+            spill = 0u;
+        }
+        const uint32_t k = turn_lanes(t0);
+        if (q.on && l < (k == 27u ? 54u : (k == 1u ? 64u : 63u))) {
+            if (k == 1u) spill |= p2g_one<PART_ALL, 1>(tile, bad, q.p, b, 0u, naff, 0u);
+            else if (k == 3u) spill |= p2g_one<PART_ALL, 3>(tile, bad, q.p, b, l % 3u, naff, 0u);
+            else if (k == 9u) spill |= p2g_one<PART_ALL, 9>(tile, bad, q.p, b, l % 9u, naff, 0u);
+            else spill |= p2g_one<PART_ALL, 27>(tile, bad, q.p, b, l % 27u, naff, 0u);
+        }
+        if (WAVE * (t0.c + 1u) >= t0.np) {
+            const uint32_t touched = wave_or_mask8(spill);
+            p2g_flush<false>(tile, bad, reinterpret_cast<float4 *>(w.stage), t0.d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+            dirty = touched == 0xFFu;
+            unlink_untouched(w, t0.d, touched, l);
+            if (CPIC && l == 0) w.binc[t0.d] = 0u;
+        }
+        t0 = t1;
+        t1 = t2;
+        q = q1;
+        slot1 = slot2;
+    }
+    if (CPIC) {
+        Turn t;
+        for (pop(1, t); t.np; pop(1, t))
+            p2g_block<CPIC, false>(w, t.d, t.np, t.v, l, tile, bad, naff, fdst, words, dirty);
+    }
+    bool first = true;
+    dirty = true;
+    for (uint32_t d = begin; d < end; ++d) {
+        const uint32_t np = ld_uniform(w.bnp + d);
+        if (np <= TEAM_MIN) continue;
+        const int4 v = ld_uniform(w.bvid + d);
+        if (v.x == OVERFLOW_VID) continue;
+        if (first) __syncthreads();   // the first wave has left its tile
+        first = false;
+        p2g_block<CPIC, true>(w, d, np, v, threadIdx.x, tiles[0], bads[0], naffs[0], fdst, words, dirty);
     }
 }
 
@@ -1246,10 +1441,11 @@ struct GatherGrid {
     }
 };
 
-// Returns the position and flags it wrote (xo, flo), for the caller's key insertion.
+// Returns the position, flags and bound codes of what it wrote (xo, flo, codes), for the
+// caller's key insertion.
 template <class Gather, bool CPIC>
 __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, uint32_t d, Gather &gather, f3 &xo,
-                                             uint32_t &flo)
+                                             uint32_t &flo, uint32_t &codes)
 {
     {
         const uint32_t slot = w.perm[pos];
@@ -1458,6 +1654,7 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
         w.out.uplane(PID)[pos] = id;
         xo = npos;
         flo = fl;
+        codes = fl & FLAG_ENABLED ? bound_codes(vel, C, mass, sc.h) : 0u;
     }
 }
 
@@ -1676,15 +1873,15 @@ __global__ void __launch_bounds__(g2p_threads<CPIC>()) k_g2p_update(WorldDev w)
     const uint32_t pos = pbegin + threadIdx.x;
     bool valid = pos < pend;
     f3 xo = mk3(0, 0, 0);
-    uint32_t flo = 0u;
+    uint32_t flo = 0u, codes = 0u;
     if (valid) {
         const uint32_t d = w.sblock[pos];
         if (CPIC && contact_particle(w, pos, d)) valid = false;   // keyed by k_g2p_contact
-        else g2p_particle<GatherGrid, false>(w, pos, d, grid, xo, flo);
+        else g2p_particle<GatherGrid, false>(w, pos, d, grid, xo, flo, codes);
     }
     if (pbegin + (threadIdx.x & ~(uint32_t)(WAVE - 1)) < pend) {   // the wave holds positions
         const uint32_t s = valid ? flags_scene(flo) : 0u;
-        touch_keys(w, pos, valid, s, xo.x, xo.y, xo.z);
+        touch_keys(w, pos, valid, s, xo.x, xo.y, xo.z, codes);
         if (ADAPT) next_dt_bound(w, pos, valid, s);
     }
     prepare_next_sort(w);
@@ -1700,24 +1897,26 @@ __global__ void __launch_bounds__(256) k_g2p_contact(WorldDev w)
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t pos = w.clist[i];
         f3 xo;
-        uint32_t flo;
-        g2p_particle<GatherGrid, true>(w, pos, w.sblock[pos], grid, xo, flo);
+        uint32_t flo, codes;
+        g2p_particle<GatherGrid, true>(w, pos, w.sblock[pos], grid, xo, flo, codes);
+        w.prank[pos] = codes;   // touch_keys below writes it again
     }
     const uint32_t l = lane_id();
     for (uint32_t base = blockIdx.x * blockDim.x + (threadIdx.x & ~(uint32_t)(WAVE - 1)); base < n;
          base += gridDim.x * blockDim.x) {
         const uint32_t i = base + l;
         const bool valid = i < n;
-        uint32_t pos = 0, s = 0;
+        uint32_t pos = 0, s = 0, codes = 0u;
         float x = 0.0f, y = 0.0f, z = 0.0f;
         if (valid) {
             pos = w.clist[i];
+            codes = w.prank[pos];
             s = w.bscene[w.sblock[pos]];
             x = w.out.plane(PX)[pos];
             y = w.out.plane(PY)[pos];
             z = w.out.plane(PZ)[pos];
         }
-        touch_keys(w, pos, valid, s, x, y, z);
+        touch_keys(w, pos, valid, s, x, y, z, codes);
         if (ADAPT) next_dt_bound(w, pos, valid, s);
     }
 }
@@ -2070,15 +2269,18 @@ void launch_substep(const WorldDev &w, const LaunchConfig &lc, hipStream_t st, h
     const int bscan = std::min((int)((w.b_total + btile - 1) / btile), cap);
     k_scan<MODE_COUNTS><<<std::max(bscan, 1), 256, 0, st>>>(w);
     k_scatter<<<grid_for(lc.p_hint, T, cap), T, 0, st>>>(w);
+    // Workgroups of one wave, one block each (blocks with 4 particles or more).
+    if (lc.order) k_cell_order<<<grid_for(std::min<uint64_t>(w.b_total, lc.p_hint), 1, 16 * cap), WAVE, 0, st>>>(w);
     if (ev) (void)hipEventRecord(ev[1], st);
+    const int pg = lc.p2g_blocks;
     if (w.any_cpic) {
         // CPIC worlds: the contact distance fields, then the CPIC variants of the
         // transfers (scenes without CPIC take the plain path inside them).
         if (w.n_rp) k_mesh_cdf<<<grid_for(w.n_rp, T, cap), T, 0, st>>>(w);
         k_grid_cdf<<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);   // one wave per block
         k_particle_cdf<<<grid_for(lc.p_hint, T, cap), T, 0, st>>>(w);
-        if (ev) hipExtLaunchKernelGGL(k_p2g<true>, dim3(lc.p2g_blocks), dim3(64), 0, st, ev[5], ev[6], 0, w);
-        else k_p2g<true><<<lc.p2g_blocks, 64, 0, st>>>(w);
+        if (ev) hipExtLaunchKernelGGL(k_p2g<true>, dim3(pg), dim3(P2G_WAVES * WAVE), 0, st, ev[5], ev[6], 0, w);
+        else k_p2g<true><<<pg, P2G_WAVES * WAVE, 0, st>>>(w);
         if (ev) (void)hipEventRecord(ev[2], st);
         if (w.mesh_pass) k_grid_update<true, true><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
         else k_grid_update<true, false><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
@@ -2104,8 +2306,8 @@ void launch_substep(const WorldDev &w, const LaunchConfig &lc, hipStream_t st, h
         }
         k_integrate_colliders<<<std::max(1, (int)((w.s_count * 16u + T - 1) / T)), T, 0, st>>>(w);
     } else {
-        if (ev) hipExtLaunchKernelGGL(k_p2g<false>, dim3(lc.p2g_blocks), dim3(64), 0, st, ev[5], ev[6], 0, w);
-        else k_p2g<false><<<lc.p2g_blocks, 64, 0, st>>>(w);
+        if (ev) hipExtLaunchKernelGGL(k_p2g<false>, dim3(pg), dim3(P2G_WAVES * WAVE), 0, st, ev[5], ev[6], 0, w);
+        else k_p2g<false><<<pg, P2G_WAVES * WAVE, 0, st>>>(w);
         if (ev) (void)hipEventRecord(ev[2], st);
         if (w.mesh_pass) k_grid_update<false, true><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
         else k_grid_update<false, false><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
