@@ -525,6 +525,29 @@ struct Slot {
     SlotState state = SLOT_FREE;
 };
 
+// Particles [first, first + count) of a scene as the arena's quads (quad q of particle i at
+// f[4 (q count + i)]), for the world slot `slot`.
+static void pack_particles(const HostParticles &hp, size_t first, size_t count, uint32_t slot, float *f)
+{
+    for (size_t i = 0; i < count; ++i) {
+        const size_t k = first + i;
+        float row[NUM_PLANES];
+        uint32_t flags = make_flags(hp.enabled[k] != 0, hp.fixed[k] != 0, hp.cls[k], slot), id = (uint32_t)k;
+        std::memcpy(row + PX, &hp.x[3 * k], 12);
+        std::memcpy(row + PFLAGS, &flags, 4);
+        std::memcpy(row + PVX, &hp.v[3 * k], 12);
+        std::memcpy(row + PAFF, &hp.aff[k], 4);
+        std::memcpy(row + PC0, &hp.C[9 * k], 36);
+        row[PMASS] = hp.mass[k];
+        row[PVOL0] = hp.vol0[k];
+        std::memcpy(row + PID, &id, 4);
+        std::memcpy(row + PF0, &hp.F[9 * k], 36);
+        std::memcpy(row + PS0, &hp.pstate[3 * k], 12);
+        std::memcpy(row + PNX, &hp.cdf[4 * k], 16);
+        for (int q = 0; q < NUM_QUADS; ++q) std::memcpy(f + 4 * (q * count + i), row + 4 * q, 16);
+    }
+}
+
 class World {
   public:
     explicit World(nxm_ctx *ctx) : ctx_(ctx) {}
@@ -634,19 +657,16 @@ class World {
             if (st != NXM_OK) return st;
         }
         const HostParticles &hp = sc->hp;
-        constexpr int NUP = NUM_PLANES;
         if (sc->staged_chunk >= 0) {
             if (first == 0 && count == sc->staged_n) {
                 // Packed by nxm_scene_stage_upload: add the world slot to the flags and queue.
                 const int k = sc->staged_chunk;
                 float *f = reinterpret_cast<float *>(sc->ctx->pool.ptr(k));
-                uint32_t *uf = reinterpret_cast<uint32_t *>(f + (size_t)PFLAGS * count);
+                uint32_t *uf = reinterpret_cast<uint32_t *>(f) + PFLAGS;   // in the first quad
                 const uint32_t sbits = sc->slot << 16;
-                for (size_t i = 0; i < count; ++i) uf[i] |= sbits;
-                Arena a = arena(cur_);
+                for (size_t i = 0; i < count; ++i) uf[4 * i] |= sbits;
                 const uint32_t at = p_in_;
-                for (int p = 0; p < NUP; ++p)
-                    HIP_TRY(hipMemcpyAsync(a.plane(p) + at, f + (size_t)p * count, count * 4, hipMemcpyHostToDevice, stream_));
+                HIP_TRY(put_quads(f, at, count));
                 sc->staged_chunk = -1;
                 HIP_TRY(sc->ctx->pool.give(k, stream_));
                 sc->ranges.push_back(SceneRange{at, (uint32_t)count});
@@ -660,37 +680,28 @@ class World {
         }
         char *stage = nullptr;
         size_t ci = 0;
-        nxm_status st = pinned(NUP * count * 4, &stage, &ci);
+        nxm_status st = pinned(NUM_PLANES * count * 4, &stage, &ci);
         if (st != NXM_OK) return st;
         float *f = reinterpret_cast<float *>(stage);
-        auto put = [&](int p, const float *src, int stride, int comp) {
-            float *dst = f + (size_t)p * count;
-            for (size_t i = 0; i < count; ++i) dst[i] = src[(first + i) * stride + comp];
-        };
-        for (int c = 0; c < 3; ++c) put(PX + c, hp.x.data(), 3, c);
-        for (int c = 0; c < 3; ++c) put(PVX + c, hp.v.data(), 3, c);
-        for (int c = 0; c < 9; ++c) put(PC0 + c, hp.C.data(), 9, c);
-        for (int c = 0; c < 9; ++c) put(PF0 + c, hp.F.data(), 9, c);
-        put(PMASS, hp.mass.data(), 1, 0);
-        put(PVOL0, hp.vol0.data(), 1, 0);
-        for (int c = 0; c < 3; ++c) put(PS0 + c, hp.pstate.data(), 3, c);
-        std::memcpy(f + (size_t)PAFF * count, hp.aff.data() + first, count * 4);
-        for (int c = 0; c < 4; ++c) put(PNX + c, hp.cdf.data(), 4, c);
-        uint32_t *uf = reinterpret_cast<uint32_t *>(f + (size_t)PFLAGS * count);
-        uint32_t *ui = reinterpret_cast<uint32_t *>(f + (size_t)PID * count);
-        for (size_t i = 0; i < count; ++i) {
-            uf[i] = make_flags(hp.enabled[first + i] != 0, hp.fixed[first + i] != 0, hp.cls[first + i], sc->slot);
-            ui[i] = (uint32_t)(first + i);
-        }
-        Arena a = arena(cur_);
+        pack_particles(hp, first, count, sc->slot, f);
         const uint32_t at = p_in_;
-        for (int p = 0; p < NUP; ++p)
-            HIP_TRY(hipMemcpyAsync(a.plane(p) + at, f + (size_t)p * count, count * 4, hipMemcpyHostToDevice, stream_));
+        HIP_TRY(put_quads(f, at, count));
         HIP_TRY(hipEventRecord(pins_[ci].ev, stream_));
         sc->ranges.push_back(SceneRange{at, (uint32_t)count});
         p_in_ += (uint32_t)count;
         pin_dirty_ = true;
         return NXM_OK;
+    }
+
+    // Queues the copies of packed quads to positions [at, at + count) of the next step's input.
+    hipError_t put_quads(const float *f, uint32_t at, size_t count)
+    {
+        for (int q = 0; q < NUM_QUADS; ++q) {
+            const hipError_t e = hipMemcpyAsync(arena(cur_).quad(q) + at, f + 4 * q * count, count * 16,
+                                                hipMemcpyHostToDevice, stream_);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
     }
 
     // Detaches a scene whose state is discarded (the scene is being destroyed): no copy.
@@ -753,9 +764,9 @@ class World {
     };
 
     // Reads rows of the scene's particles in id order: gathered on the device into the arena
-    // that the next step will write (its position planes stay: the canonical sort reads
-    // them), then copied through two pinned chunks, one being filled while the other is
-    // taken (copy_out).  At most 33 words a particle.  Synchronizes; the errors latched so
+    // that the next step will write (its first quad, the positions, stays: the canonical
+    // sort reads it), then copied through two pinned halves, one being filled while the
+    // other is taken (copy_out).  At most 32 words a particle.  Synchronizes; the errors latched so
     // far are reported before anything is written.
     nxm_status read_rows(nxm_scene *sc, std::initializer_list<ReadItem> items)
     {
@@ -771,8 +782,8 @@ class World {
             words += n * it.comps;
         }
         if (words == 0) return sync();
-        if (words > (size_t)(NUM_PLANES - PVX) * p_cap_) return fail(NXM_ERR_INVALID_ARGUMENT, "readback too wide");
-        float *dev = arena(cur_ ^ 1).plane(PVX);
+        if (words > (size_t)(NUM_PLANES - 4) * p_cap_) return fail(NXM_ERR_INVALID_ARGUMENT, "readback too wide");
+        float *dev = reinterpret_cast<float *>(arena(cur_ ^ 1).quad(1));
         for (const SceneRange &r : sc->ranges)
             launch_read_rows(arena(cur_), r.start, r.count, list, dev, (int)ctx_->num_cus * 8, stream_);
         HIP_TRY(hipGetLastError());
@@ -1069,7 +1080,7 @@ class World {
         const HostParticles &hp = sc->hp;
         // The records and the constant properties they use lie in the arena that the next
         // step will write, as in read_rows (24 + 3 words a particle).
-        float *dout = arena(cur_ ^ 1).plane(PVX), *props = dout + 24 * n;
+        float *dout = reinterpret_cast<float *>(arena(cur_ ^ 1).quad(1)), *props = dout + 24 * n;
         uint32_t *group = reinterpret_cast<uint32_t *>(props + 2 * n);
         if (npal > read_palette_.n) {
             nxm_status st = sync();   // a call in flight may read the one that is replaced
@@ -1138,7 +1149,9 @@ class World {
         // particles of the scene: its output range
         for (const SceneRange &r : sc->ranges) {
             std::vector<uint32_t> ids(r.count), sb(r.count), pc(r.count);
-            HIP_TRY(hipMemcpy(ids.data(), arena(cur_).uplane(PID) + r.start, r.count * 4, hipMemcpyDeviceToHost));
+            std::vector<float4> quad(r.count);   // the one that holds the ids
+            HIP_TRY(hipMemcpy(quad.data(), arena(cur_).quad(PID >> 2) + r.start, r.count * 16, hipMemcpyDeviceToHost));
+            for (uint32_t i = 0; i < r.count; ++i) std::memcpy(&ids[i], reinterpret_cast<float *>(&quad[i]) + (PID & 3), 4);
             HIP_TRY(hipMemcpy(sb.data(), sblock_.p + r.start, r.count * 4, hipMemcpyDeviceToHost));
             HIP_TRY(hipMemcpy(pc.data(), pcell.p + r.start, r.count * 4, hipMemcpyDeviceToHost));
             for (uint32_t i = 0; i < r.count; ++i) {
@@ -1250,7 +1263,7 @@ class World {
         return NXM_OK;
     }
 
-    Arena arena(int k) const { return Arena{arenas_[k].p, p_cap_}; }
+    Arena arena(int k) const { return Arena{reinterpret_cast<float4 *>(arenas_[k].p), p_cap_}; }
 
     WorldDev view() const
     {
@@ -1285,9 +1298,9 @@ class World {
         HIP_TRY(na[0].reserve((size_t)NUM_PLANES * cap));
         HIP_TRY(na[1].reserve((size_t)NUM_PLANES * cap));
         if (p_in_) {
-            for (int p = 0; p < NUM_PLANES; ++p)
-                HIP_TRY(hipMemcpy(na[cur_].p + (size_t)p * cap, arenas_[cur_].p + (size_t)p * p_cap_, (size_t)p_in_ * 4,
-                                  hipMemcpyDeviceToDevice));
+            for (int q = 0; q < NUM_QUADS; ++q)
+                HIP_TRY(hipMemcpy(na[cur_].p + 4 * (size_t)q * cap, arenas_[cur_].p + 4 * (size_t)q * p_cap_,
+                                  (size_t)p_in_ * 16, hipMemcpyDeviceToDevice));
         }
         for (int k = 0; k < 2; ++k) {
             arenas_[k].release();
@@ -2095,25 +2108,7 @@ nxm_status nxm_scene_stage_upload(nxm_scene *sc)
     char *buf = nullptr;
     HIP_TRY(sc->ctx->pool.take((size_t)NUM_PLANES * n * 4, &k, &buf));
     float *f = reinterpret_cast<float *>(buf);
-    auto put = [&](int p, const float *src, int stride, int comp) {
-        float *dst = f + (size_t)p * n;
-        for (size_t i = 0; i < n; ++i) dst[i] = src[i * stride + comp];
-    };
-    for (int c = 0; c < 3; ++c) put(PX + c, hp.x.data(), 3, c);
-    for (int c = 0; c < 3; ++c) put(PVX + c, hp.v.data(), 3, c);
-    for (int c = 0; c < 9; ++c) put(PC0 + c, hp.C.data(), 9, c);
-    for (int c = 0; c < 9; ++c) put(PF0 + c, hp.F.data(), 9, c);
-    put(PMASS, hp.mass.data(), 1, 0);
-    put(PVOL0, hp.vol0.data(), 1, 0);
-    for (int c = 0; c < 3; ++c) put(PS0 + c, hp.pstate.data(), 3, c);
-    std::memcpy(f + (size_t)PAFF * n, hp.aff.data(), n * 4);
-    for (int c = 0; c < 4; ++c) put(PNX + c, hp.cdf.data(), 4, c);
-    uint32_t *uf = reinterpret_cast<uint32_t *>(f + (size_t)PFLAGS * n);
-    uint32_t *ui = reinterpret_cast<uint32_t *>(f + (size_t)PID * n);
-    for (size_t i = 0; i < n; ++i) {
-        uf[i] = make_flags(hp.enabled[i] != 0, hp.fixed[i] != 0, hp.cls[i], 0u);
-        ui[i] = (uint32_t)i;
-    }
+    pack_particles(hp, 0, n, 0u, f);
     sc->staged_chunk = k;
     sc->staged_n = n;
     return NXM_OK;
@@ -2704,8 +2699,8 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     char *base = static_cast<char *>(ctx->scratch);
     auto at = [&](size_t off) { return static_cast<void *>(base + off); };
     WorldDev w{};
-    w.in = Arena{static_cast<float *>(at(o_arena0)), p_cap};
-    w.out = Arena{static_cast<float *>(at(o_arena1)), p_cap};
+    w.in = Arena{static_cast<float4 *>(at(o_arena0)), p_cap};
+    w.out = Arena{static_cast<float4 *>(at(o_arena1)), p_cap};
     w.pkey = static_cast<uint32_t *>(at(o_pkey)); w.pdense = static_cast<uint32_t *>(at(o_pdense));
     w.prank = static_cast<uint32_t *>(at(o_prank)); w.perm = static_cast<uint32_t *>(at(o_perm));
     w.sblock = static_cast<uint32_t *>(at(o_sblock));

@@ -32,24 +32,37 @@ __host__ __device__ inline uint32_t make_flags(bool enabled, bool fixed, uint32_
 constexpr uint32_t MAX_CLASSES = 1u << 14;
 constexpr uint32_t MAX_SCENES = 1u << 16;
 
-// Particle arena planes (structure of arrays, one f32/u32 plane per component).
+// Particle arena: NUM_PLANES words per particle in groups of four (quads), each quad an array
+// of float4 over the particles, so that a particle's words are read and written 16 bytes at
+// a time.  With a plane per word P2G read a particle by 17 loads of 4 bytes and G2P by 20,
+// writing 28: their addresses alone filled the scalar registers.  Quads:
+//   0  position, flags          3  C4 .. C7                     6  F4 .. F7
+//   1  velocity, affinity       4  C8, mass, volume, id         7  F8, plastic state
+//   2  C0 .. C3                 5  F0 .. F3                     8  contact normal, distance
 enum Plane : int {
-    PX = 0, PY, PZ,
-    PVX, PVY, PVZ,
-    PC0, PC1, PC2, PC3, PC4, PC5, PC6, PC7, PC8,   // affine, column-major
-    PF0, PF1, PF2, PF3, PF4, PF5, PF6, PF7, PF8,   // deformation gradient, column-major
-    PMASS, PVOL0,
+    PX = 0, PY, PZ, PFLAGS,
+    PVX, PVY, PVZ, PAFF,                            // PAFF: CPIC affinity word
+    PC0, PC1, PC2, PC3, PC4, PC5, PC6, PC7, PC8,    // affine, column-major
+    PMASS, PVOL0, PID,
+    PF0, PF1, PF2, PF3, PF4, PF5, PF6, PF7, PF8,    // deformation gradient, column-major
     PS0, PS1, PS2,                                  // plastic state (sand: 3 words, snow: 1)
-    PAFF, PNX, PNY, PNZ, PSD,                       // CPIC: affinity word, contact normal, signed distance
-    PFLAGS, PID,
+    PNX, PNY, PNZ, PSD,                             // CPIC: contact normal, signed distance
     NUM_PLANES
 };
+constexpr int NUM_QUADS = NUM_PLANES / 4;
+static_assert(NUM_PLANES % 4 == 0, "whole quads");
 
 struct Arena {
-    float *base;       // NUM_PLANES planes of `stride` elements
+    float4 *base;      // NUM_QUADS arrays of `stride` quads
     uint32_t stride;
-    __device__ __host__ float *plane(int p) const { return base + (size_t)p * stride; }
-    __device__ __host__ uint32_t *uplane(int p) const { return reinterpret_cast<uint32_t *>(base + (size_t)p * stride); }
+    // One word of every particle: element i is particle i's.
+    template <class T> struct Words {
+        T *p;
+        __device__ __host__ T &operator[](size_t i) const { return p[4 * i]; }
+    };
+    __device__ __host__ float4 *quad(int q) const { return base + (size_t)q * stride; }
+    __device__ __host__ Words<float> plane(int p) const { return {reinterpret_cast<float *>(quad(p >> 2)) + (p & 3)}; }
+    __device__ __host__ Words<uint32_t> uplane(int p) const { return {reinterpret_cast<uint32_t *>(quad(p >> 2)) + (p & 3)}; }
 };
 
 // One scene of a world.

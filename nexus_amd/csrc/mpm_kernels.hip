@@ -150,17 +150,21 @@ struct P2GIn {
     float px, py, pz, m;
     f3 v;
     m3 C;
+    uint32_t flags;
 };
 
 __device__ inline P2GIn p2g_load(const WorldDev &w, uint32_t slot)
 {
+    const float4 q0 = w.in.quad(0)[slot], q1 = w.in.quad(1)[slot], q2 = w.in.quad(2)[slot], q3 = w.in.quad(3)[slot],
+                 q4 = w.in.quad(4)[slot];
     P2GIn p;
-    p.px = w.in.plane(PX)[slot]; p.py = w.in.plane(PY)[slot]; p.pz = w.in.plane(PZ)[slot];
-    p.m = w.in.plane(PMASS)[slot];
-    p.v = mk3(w.in.plane(PVX)[slot], w.in.plane(PVY)[slot], w.in.plane(PVZ)[slot]);
-    p.C.c0 = mk3(w.in.plane(PC0)[slot], w.in.plane(PC1)[slot], w.in.plane(PC2)[slot]);
-    p.C.c1 = mk3(w.in.plane(PC3)[slot], w.in.plane(PC4)[slot], w.in.plane(PC5)[slot]);
-    p.C.c2 = mk3(w.in.plane(PC6)[slot], w.in.plane(PC7)[slot], w.in.plane(PC8)[slot]);
+    p.px = q0.x; p.py = q0.y; p.pz = q0.z;
+    p.flags = __float_as_uint(q0.w);
+    p.v = mk3(q1.x, q1.y, q1.z);
+    p.C.c0 = mk3(q2.x, q2.y, q2.z);
+    p.C.c1 = mk3(q2.w, q3.x, q3.y);
+    p.C.c2 = mk3(q3.z, q3.w, q4.x);
+    p.m = q4.y;
     return p;
 }
 
@@ -190,7 +194,7 @@ __device__ inline uint32_t bound_codes(f3 v, const m3 &C, float m, float h)
 }
 
 // Block key of particle slot i at position (x, y, z) of active scene s (written to
-// pkey[i]) and its bound codes (to prank[i]), and the wave's block insertions: adjacent lanes with the same (scene, key)
+// pkey[i]), its bound codes (to prank[i]) and its scene (to pdense[i]), and the wave's block insertions: adjacent lanes with the same (scene, key)
 // form a run; each run inserts its block (marked primary) and the block's 7 +1
 // neighbours (the active set is P + {0,1}^3, src_mpm/grid/grid.rs:193-200).  Called by
 // every lane of a wave together (invalid lanes with valid = false), so that the lanes'
@@ -215,6 +219,7 @@ __device__ inline void touch_keys(const WorldDev &w, uint32_t i, bool valid, uin
         }
         w.pkey[i] = key;
         w.prank[i] = codes;
+        w.pdense[i] = s;
     }
     const uint32_t pk = __shfl_up(key, 1, WAVE);
     const uint32_t ps = __shfl_up(s, 1, WAVE);
@@ -266,24 +271,20 @@ __global__ void k_keys_touch(WorldDev w)
     mark_overflow_slots(w);
     const uint32_t n = w.g->p_in;
     const uint32_t nr = (n + WAVE - 1) / WAVE * WAVE;
-    const float *X = w.in.plane(PX), *Y = w.in.plane(PY), *Z = w.in.plane(PZ);
-    const uint32_t *FL = w.in.uplane(PFLAGS);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nr; i += gridDim.x * blockDim.x) {
         bool valid = i < n;
         uint32_t s = 0;
         float x = 0.0f, y = 0.0f, z = 0.0f;
         uint32_t codes = 0u;
         if (valid) {
-            const uint32_t fl = FL[i];
-            s = flags_scene(fl);
+            const P2GIn p = p2g_load(w, i);
+            s = flags_scene(p.flags);
             valid = w.scenes[s].active != 0u;
-            x = X[i];
-            y = Y[i];
-            z = Z[i];
-            if (valid && (fl & FLAG_ENABLED)) {
-                const P2GIn p = p2g_load(w, i);
-                codes = bound_codes(p.v, p.C, p.m, w.scenes[s].h);
-            }
+            if (!valid) w.pdense[i] = s;   // the count kernel leaves it out
+            x = p.px;
+            y = p.py;
+            z = p.pz;
+            if (p.flags & FLAG_ENABLED) codes = bound_codes(p.v, p.C, p.m, w.scenes[s].h);
         }
         touch_keys(w, i, valid, s, x, y, z, codes);
     }
@@ -562,12 +563,11 @@ __device__ inline void count_part(const WorldDev &w)
     const uint32_t n = w.g->p_in;
     const uint32_t nr = (n + WAVE - 1) / WAVE * WAVE;
     const uint32_t l = lane_id();
-    const uint32_t *FL = w.in.uplane(PFLAGS);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nr; i += gridDim.x * blockDim.x) {
         bool valid = i < n;
         uint32_t d = NONE, codes = 0u;
         if (valid) {
-            uint32_t s = flags_scene(FL[i]);
+            const uint32_t s = w.pdense[i];
             const SceneDev sc = w.scenes[s];
             valid = sc.active != 0u;
             if (valid) {
@@ -579,8 +579,8 @@ __device__ inline void count_part(const WorldDev &w)
                     d = w.hvals[sc.h_base + sc.h_cap];   // the overflow block: P2G does not take it
                     codes = 0u;
                 }
-                w.pdense[i] = d;
             }
+            w.pdense[i] = d;   // NONE: of a scene that has left
         }
         uint32_t pd = __shfl_up(d, 1, WAVE);
         bool pv = __shfl_up((int)valid, 1, WAVE) != 0;
@@ -644,11 +644,9 @@ __device__ inline void p2g_split(const WorldDev &w)
 __global__ void k_scatter(WorldDev w)
 {
     const uint32_t n = w.g->p_in;
-    const uint32_t *FL = w.in.uplane(PFLAGS);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        uint32_t s = flags_scene(FL[i]);
-        if (!w.scenes[s].active) continue;
-        uint32_t d = w.pdense[i];
+        const uint32_t d = w.pdense[i];
+        if (d == NONE) continue;
         uint32_t pos = w.bfirst[d] + w.prank[i];
         w.perm[pos] = i;
         w.sblock[pos] = d;
@@ -685,7 +683,8 @@ __global__ void __launch_bounds__(WAVE) k_cell_order(WorldDev w)
             #pragma unroll
             for (int k = 0; k < ORDER_PER; ++k) {
                 if (slot[k] == NONE) continue;
-                const float x = w.in.plane(PX)[slot[k]], y = w.in.plane(PY)[slot[k]], z = w.in.plane(PZ)[slot[k]];
+                const float4 q = w.in.quad(0)[slot[k]];
+                const float x = q.x, y = q.y, z = q.z;
                 // base cell in the block, 0..3 on each axis (a position without one: any cell)
                 const int cx = (int)round_div(x, sc.h, sc.inv_h) - 1 - 4 * v.x;
                 const int cy = (int)round_div(y, sc.h, sc.inv_h) - 1 - 4 * v.y;
@@ -1094,8 +1093,8 @@ __device__ __forceinline__ P2GLane p2g_fetch(const WorldDev &w, uint32_t slot)
 {
     P2GLane r{};
     if (slot != NONE) {
-        r.on = (w.in.uplane(PFLAGS)[slot] & FLAG_ENABLED) != 0u;
         r.p = p2g_load(w, slot);
+        r.on = (r.p.flags & FLAG_ENABLED) != 0u;
     }
     return r;
 }
@@ -1452,25 +1451,23 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
         const uint32_t s = w.bscene[d];
         const SceneDev sc = w.scenes[s];
         const int4 bv = w.bvid[d];
-        uint32_t fl = w.in.uplane(PFLAGS)[slot];
-        const float px = w.in.plane(PX)[slot], py = w.in.plane(PY)[slot], pz = w.in.plane(PZ)[slot];
-        float mass = w.in.plane(PMASS)[slot];
-        const float vol0 = w.in.plane(PVOL0)[slot];
-        const uint32_t id = w.in.uplane(PID)[slot];
+        const float4 q0 = w.in.quad(0)[slot], q4 = w.in.quad(4)[slot], q5 = w.in.quad(5)[slot], q6 = w.in.quad(6)[slot],
+                     q7 = w.in.quad(7)[slot];
+        uint32_t fl = __float_as_uint(q0.w);
+        const float px = q0.x, py = q0.y, pz = q0.z;
+        float mass = q4.y;
+        const float vol0 = q4.z, id = q4.w;
         m3 F;
-        F.c0 = mk3(w.in.plane(PF0)[slot], w.in.plane(PF1)[slot], w.in.plane(PF2)[slot]);
-        F.c1 = mk3(w.in.plane(PF3)[slot], w.in.plane(PF4)[slot], w.in.plane(PF5)[slot]);
-        F.c2 = mk3(w.in.plane(PF6)[slot], w.in.plane(PF7)[slot], w.in.plane(PF8)[slot]);
+        F.c0 = mk3(q5.x, q5.y, q5.z);
+        F.c1 = mk3(q5.w, q6.x, q6.y);
+        F.c2 = mk3(q6.z, q6.w, q7.x);
+        // Per-particle plastic state: three words for the sand tags, one for snow.
+        float ps0 = q7.y, ps1 = q7.z, ps2 = q7.w;
         f3 vel;
         m3 C;
         f3 npos = mk3(px, py, pz);
         const ClassDev &cls = w.classes[sc.class_base + flags_class(fl)];
         const uint32_t tag = cls.tag;
-        // Per-particle plastic state: three words for the sand tags, one for snow.
-        const bool sand = tag == 2u || tag == 3u, snow = tag == 5u;
-        float ps0 = 0.0f, ps1 = 0.0f, ps2 = 0.0f;
-        if (sand || snow) ps0 = w.in.plane(PS0)[slot];
-        if (sand) { ps1 = w.in.plane(PS1)[slot]; ps2 = w.in.plane(PS2)[slot]; }
         // CPIC: this substep's particle contact field (written at the sorted position).  A
         // particle without affinity bits is compatible with every node and its contact
         // field is zero (a regular fit needs a node sharing an affinity), so it takes the
@@ -1638,20 +1635,15 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
                 npos = mk3(px, py, pz);
             }
         }
-        w.out.plane(PX)[pos] = npos.x; w.out.plane(PY)[pos] = npos.y; w.out.plane(PZ)[pos] = npos.z;
-        w.out.plane(PVX)[pos] = vel.x; w.out.plane(PVY)[pos] = vel.y; w.out.plane(PVZ)[pos] = vel.z;
-        w.out.plane(PC0)[pos] = C.c0.x; w.out.plane(PC1)[pos] = C.c0.y; w.out.plane(PC2)[pos] = C.c0.z;
-        w.out.plane(PC3)[pos] = C.c1.x; w.out.plane(PC4)[pos] = C.c1.y; w.out.plane(PC5)[pos] = C.c1.z;
-        w.out.plane(PC6)[pos] = C.c2.x; w.out.plane(PC7)[pos] = C.c2.y; w.out.plane(PC8)[pos] = C.c2.z;
-        w.out.plane(PF0)[pos] = F.c0.x; w.out.plane(PF1)[pos] = F.c0.y; w.out.plane(PF2)[pos] = F.c0.z;
-        w.out.plane(PF3)[pos] = F.c1.x; w.out.plane(PF4)[pos] = F.c1.y; w.out.plane(PF5)[pos] = F.c1.z;
-        w.out.plane(PF6)[pos] = F.c2.x; w.out.plane(PF7)[pos] = F.c2.y; w.out.plane(PF8)[pos] = F.c2.z;
-        w.out.plane(PMASS)[pos] = mass;
-        w.out.plane(PVOL0)[pos] = vol0;
-        if (sand || snow) w.out.plane(PS0)[pos] = ps0;
-        if (sand) { w.out.plane(PS1)[pos] = ps1; w.out.plane(PS2)[pos] = ps2; }
-        w.out.uplane(PFLAGS)[pos] = fl;
-        w.out.uplane(PID)[pos] = id;
+        w.out.quad(0)[pos] = make_float4(npos.x, npos.y, npos.z, __uint_as_float(fl));
+        // The affinity word beside the velocity is this substep's own (k_particle_cdf).
+        *reinterpret_cast<f3 *>(&w.out.quad(1)[pos]) = vel;
+        w.out.quad(2)[pos] = make_float4(C.c0.x, C.c0.y, C.c0.z, C.c1.x);
+        w.out.quad(3)[pos] = make_float4(C.c1.y, C.c1.z, C.c2.x, C.c2.y);
+        w.out.quad(4)[pos] = make_float4(C.c2.z, mass, vol0, id);
+        w.out.quad(5)[pos] = make_float4(F.c0.x, F.c0.y, F.c0.z, F.c1.x);
+        w.out.quad(6)[pos] = make_float4(F.c1.y, F.c1.z, F.c2.x, F.c2.y);
+        w.out.quad(7)[pos] = make_float4(F.c2.z, ps0, ps1, ps2);
         xo = npos;
         flo = fl;
         codes = fl & FLAG_ENABLED ? bound_codes(vel, C, mass, sc.h) : 0u;
@@ -2486,16 +2478,7 @@ __global__ void k_noalloc_pack(WorldDev w, NoallocTables t, NoallocParticles p)
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = blockIdx.x * blockDim.x + tid; i < t.n; i += gridDim.x * blockDim.x) {
         const Arena a = w.in;
-        for (int c = 0; c < 3; ++c) {
-            a.plane(PX + c)[i] = p.x[3 * (size_t)i + c];
-            a.plane(PVX + c)[i] = p.v[3 * (size_t)i + c];
-        }
-        for (int c = 0; c < 9; ++c) {
-            a.plane(PC0 + c)[i] = p.C[9 * (size_t)i + c];
-            a.plane(PF0 + c)[i] = p.F[9 * (size_t)i + c];
-        }
-        a.plane(PMASS)[i] = p.mass[i];
-        a.plane(PVOL0)[i] = p.vol0[i];
+        const float *x = p.x + 3 * (size_t)i, *v = p.v + 3 * (size_t)i, *C = p.C + 9 * (size_t)i, *F = p.F + 9 * (size_t)i;
         const uint32_t f = p.flags[i];
         uint32_t cls = flags_class(f);
         if (cls >= t.n_classes) {
@@ -2507,11 +2490,19 @@ __global__ void k_noalloc_pack(WorldDev w, NoallocTables t, NoallocParticles p)
         // three, snow's one), as an upload takes it from the particle's model words.
         const uint32_t tag = t.classes[cls].tag;
         const int pw = (tag == 2u || tag == 3u) ? 3 : tag == 5u ? 1 : 0;
+        float ps[3];
         for (int c = 0; c < 3; ++c)
-            a.plane(PS0 + c)[i] = c < pw ? (p.pstate ? p.pstate[3 * (size_t)i + c] : t.classes[cls].w[c]) : 0.0f;
-        for (int c = PAFF; c <= PSD; ++c) a.plane(c)[i] = 0.0f;
-        a.uplane(PFLAGS)[i] = make_flags((f & FLAG_ENABLED) != 0u, (f & FLAG_FIXED) != 0u, cls, 0u);
-        a.uplane(PID)[i] = i;
+            ps[c] = c < pw ? (p.pstate ? p.pstate[3 * (size_t)i + c] : t.classes[cls].w[c]) : 0.0f;
+        const uint32_t flags = make_flags((f & FLAG_ENABLED) != 0u, (f & FLAG_FIXED) != 0u, cls, 0u);
+        a.quad(0)[i] = make_float4(x[0], x[1], x[2], __uint_as_float(flags));
+        a.quad(1)[i] = make_float4(v[0], v[1], v[2], 0.0f);
+        a.quad(2)[i] = make_float4(C[0], C[1], C[2], C[3]);
+        a.quad(3)[i] = make_float4(C[4], C[5], C[6], C[7]);
+        a.quad(4)[i] = make_float4(C[8], p.mass[i], p.vol0[i], __uint_as_float(i));
+        a.quad(5)[i] = make_float4(F[0], F[1], F[2], F[3]);
+        a.quad(6)[i] = make_float4(F[4], F[5], F[6], F[7]);
+        a.quad(7)[i] = make_float4(F[8], ps[0], ps[1], ps[2]);
+        a.quad(8)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 }
 
