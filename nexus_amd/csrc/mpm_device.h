@@ -304,6 +304,7 @@ __device__ inline float rcp_hw(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline float rsq_hw(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ inline float sqrt_hw(float x) { return __builtin_amdgcn_sqrtf(x); }
 
+template <bool WITH_V>
 __device__ inline void jacobi_pair(f3 &ap, f3 &aq, f3 &vp, f3 &vq, float &off)
 {
     float alpha = dot(ap, ap), beta = dot(aq, aq), gamma = dot(ap, aq);
@@ -316,9 +317,11 @@ __device__ inline void jacobi_pair(f3 &ap, f3 &aq, f3 &vp, f3 &vq, float &off)
     float t = az > 1.0e15f ? 0.5f * rcp_hw(zeta) : copysignf(rcp_hw(az + sqrt_hw(1.0f + zeta * zeta)), zeta);
     float c = rsq_hw(1.0f + t * t);
     float s = c * t;
-    f3 a0 = ap, a1 = aq, w0 = vp, w1 = vq;
+    f3 a0 = ap, a1 = aq;
     ap = a0 * c - a1 * s;
     aq = a0 * s + a1 * c;
+    if (!WITH_V) return;
+    f3 w0 = vp, w1 = vq;
     vp = w0 * c - w1 * s;
     vq = w0 * s + w1 * c;
 }
@@ -330,15 +333,16 @@ __device__ inline f3 any_orthogonal(f3 a)
     return c / length(c);
 }
 
-__device__ inline void svd3(const m3 &F, m3 &U, f3 &s, m3 &V)
+template <bool WITH_V>
+__device__ inline void svd3_parts(const m3 &F, m3 &U, f3 &s, m3 &V)
 {
     f3 a0 = F.c0, a1 = F.c1, a2 = F.c2;
     f3 w0 = mk3(1, 0, 0), w1 = mk3(0, 1, 0), w2 = mk3(0, 0, 1);
     for (int sweep = 0; sweep < 8; ++sweep) {
         float off = 0.0f;
-        jacobi_pair(a0, a1, w0, w1, off);
-        jacobi_pair(a0, a2, w0, w2, off);
-        jacobi_pair(a1, a2, w1, w2, off);
+        jacobi_pair<WITH_V>(a0, a1, w0, w1, off);
+        jacobi_pair<WITH_V>(a0, a2, w0, w2, off);
+        jacobi_pair<WITH_V>(a1, a2, w1, w2, off);
         if (!(off > 1.0e-14f)) break;
     }
     float s0 = sqrt_hw(dot(a0, a0)), s1 = sqrt_hw(dot(a1, a1)), s2 = sqrt_hw(dot(a2, a2));
@@ -367,15 +371,22 @@ __device__ inline void svd3(const m3 &F, m3 &U, f3 &s, m3 &V)
         }
     }
     U = m3{u0, u1, u2};
-    V = m3{w0, w1, w2};
+    V = m3{w0, w1, w2};   // a product of rotations
     s = mk3(s0, s1, s2);
-    if (det(V) < 0.0f) { V.c2 = V.c2 * -1.0f; U.c2 = U.c2 * -1.0f; }
     if (det(U) < 0.0f) {
         // flip the column of the smallest singular value
         if (s.x <= s.y && s.x <= s.z) { U.c0 = U.c0 * -1.0f; s.x = -s.x; }
         else if (s.y <= s.z) { U.c1 = U.c1 * -1.0f; s.y = -s.y; }
         else { U.c2 = U.c2 * -1.0f; s.z = -s.z; }
     }
+}
+
+__device__ inline void svd3(const m3 &F, m3 &U, f3 &s, m3 &V) { svd3_parts<true>(F, U, s, V); }
+// U and s alone: a quarter less work and nine registers fewer.
+__device__ inline void svd3_us(const m3 &F, m3 &U, f3 &s)
+{
+    m3 unused;
+    svd3_parts<false>(F, U, s, unused);
 }
 
 // U diag(d) U^T (symmetric), used by the corotated stress with a known SVD.
@@ -430,12 +441,21 @@ __device__ inline float dp_alpha(const float *dp, float q)
     return 0.81649658f * (2.0f * sa) * rcp_hw(3.0f - sa);   // sqrt(2/3)
 }
 
-// DruckerPragerPlasticity::project (drucker_prager.rs:224-267 with :121-167).  Updates
-// F and the plastic state {det Fp, q, log volume gain} in place; returns the SVD of
-// the projected F in (U, s, V) for the elastic backbone.
-__device__ inline void dp_project(const float *dp, float &pdet, float &q, float &lvg, m3 &F, m3 &U, f3 &s, m3 &V)
+// e^t - 1 without the cancellation at small t.
+__device__ inline float growth(float t)
 {
-    svd3(F, U, s, V);
+    if (fabsf(t) < 0.0625f) return t * (1.0f + t * (0.5f + t * (1.0f / 6.0f + t * (1.0f / 24.0f + t * (1.0f / 120.0f)))));
+    return __expf(t) - 1.0f;
+}
+
+// DruckerPragerPlasticity::project (drucker_prager.rs:224-267 with :121-167).  Updates
+// F and the plastic state {det Fp, q, log volume gain} in place, given the left singular
+// vectors U and the singular values s of F; s comes back as the projected F's.  The
+// projected F = U s' V^T is F + U diag(s' / s - 1) U^T F: no right singular vectors, and the
+// rounding of U weighs only on the change (U s' V^T, and U diag(s' / s) U^T F more so, round
+// all of F anew at every plastic substep).
+__device__ inline void dp_project(const float *dp, float &pdet, float &q, float &lvg, m3 &F, const m3 &U, f3 &s)
+{
     if (dp[4] == 0.0f) return;
     float alpha = dp_alpha(dp, q);
     const float d = 3.0f, inv_d3 = 1.0f / 3.0f;
@@ -445,27 +465,29 @@ __device__ inline void dp_project(const float *dp, float &pdet, float &q, float 
     float m = tr * inv_d3;
     f3 dev = mk3(strain.x - m, strain.y - m, strain.z - m);
     float shifted = tr - dp[6];
-    f3 ns;
+    f3 g;       // growth of the singular values, s' / s - 1
     float dq;
     if (shifted > 0.0f || (dev.x == 0.0f && dev.y == 0.0f && dev.z == 0.0f)) {
         float e = __expf(dp[6] * inv_d3);
-        ns = mk3(e, e, e);
+        g = mk3((e - s.x) * rcp_hw(s.x), (e - s.y) * rcp_hw(s.y), (e - s.z) * rcp_hw(s.z));
         dq = length(strain);
     } else {
         float dn = length(dev);
         float gamma = dn + (d * dp[4] + 2.0f * dp[5]) * rcp_hw(2.0f * dp[5]) * shifted * alpha;
         if (gamma <= 0.0f) return;   // elastic: state and F unchanged
+        // s' = exp(strain - k dev) with strain = log s + lg: s' / s = exp(lg - k dev).
         float k = gamma * rcp_hw(dn);
-        ns = mk3(__expf(strain.x - dev.x * k), __expf(strain.y - dev.y * k), __expf(strain.z - dev.z * k));
+        g = mk3(growth(lg - dev.x * k), growth(lg - dev.y * k), growth(lg - dev.z * k));
         dq = gamma;
     }
+    const f3 ns = mk3(s.x + s.x * g.x, s.y + s.y * g.y, s.z + s.z * g.z);
     float prev_det = s.x * s.y * s.z;
     float new_det = ns.x * ns.y * ns.z;
     pdet = pdet * prev_det * rcp_hw(new_det);
     lvg = lvg + __logf(prev_det) - __logf(new_det);
     q = q + dq;
+    F = F + mul(u_diag_ut(U, g), F);
     s = ns;
-    F = recompose(U, s, V);
 }
 
 // SnowPlasticity::project and hardening_factor (snow.rs:77-113), sp = {critical

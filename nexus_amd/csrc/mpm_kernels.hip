@@ -1425,18 +1425,71 @@ struct GatherGrid {
         if (blk == NONE) return NONE;
         return blk * NODES_PER_BLOCK + (tx & 3) + 4 * (ty & 3) + 16 * (tz & 3);
     }
-    // Without branches: a missing block's node reads node 0 (always allocated) and is
-    // replaced by zero, so the 27 reads of a particle go out back to back.
-    __device__ f3 at(int tx, int ty, int tz) const
+    // The quadratic transfer over the 27 nodes at base position (bx, by, bz): vel = sum w v and
+    // g_j = sum w v s_j over the offsets s, as sums along x, then y, then z of nine rows.  A
+    // row's three nodes lie in at most two blocks, picked per row, so a node costs one select
+    // and one add beside its load.  Missing blocks (a scene over its capacity) read as zero, in
+    // a loop of its own.  Against 27 nodes one by one, each with its block picked from eight
+    // and ten multiply-adds of its own, with the SVD copy without V: 141 -> 115 registers (4
+    // waves a SIMD instead of 3), the 1M sand column's G2P 102 -> 90 us (2.1 TB/s of state),
+    // 4 x 510k clumped fluid 251 -> 231, 32 mixed scenes 136 -> 123, the CPIC sand's plain
+    // particles 34 -> 28.
+    __device__ __forceinline__ void transfer(int bx, int by, int bz, const float (&wx)[3], const float (&wy)[3],
+                                             const float (&wz)[3], f3 &vel, f3 &gx, f3 &gy, f3 &gz) const
     {
-        const bool ox = tx >= 4, oy = ty >= 4, oz = tz >= 4;
-        const uint32_t z0 = oz ? n1 : n0, z1 = oz ? n3 : n2, z2 = oz ? n5 : n4, z3 = oz ? n7 : n6;
-        const uint32_t y0 = oy ? z1 : z0, y1 = oy ? z3 : z2;
-        const uint32_t blk = ox ? y1 : y0;
-        const bool none = blk == NONE;
-        const uint32_t i = none ? 0u : blk * NODES_PER_BLOCK + (tx & 3) + 4 * (ty & 3) + 16 * (tz & 3);
+        const bool whole = n0 != NONE && n1 != NONE && n2 != NONE && n3 != NONE && n4 != NONE && n5 != NONE &&
+                           n6 != NONE && n7 != NONE;
+        if (whole) sum<true>(bx, by, bz, wx, wy, wz, vel, gx, gy, gz);
+        else sum<false>(bx, by, bz, wx, wy, wz, vel, gx, gy, gz);
+    }
+    template <bool WHOLE>
+    __device__ __forceinline__ void sum(int bx, int by, int bz, const float (&wx)[3], const float (&wy)[3],
+                                        const float (&wz)[3], f3 &vel, f3 &gx, f3 &gy, f3 &gz) const
+    {
+        const bool x1 = bx == 3, x2 = bx >= 2;                       // offset 1, 2 beyond the block
+        const uint32_t lx0 = bx, lx1 = (bx + 1) & 3, lx2 = (bx + 2) & 3;
+        constexpr int WHOLLY = WHOLE ? 3 : 1;                        // (the rare case: a loop)
+        #pragma unroll WHOLLY
+        for (int sz = 0; sz < 3; ++sz) {
+            const bool oz = bz + sz >= 4;
+            const uint32_t a0 = oz ? n1 : n0, a1 = oz ? n3 : n2, b0 = oz ? n5 : n4, b1 = oz ? n7 : n6;
+            const uint32_t lz = 16u * ((bz + sz) & 3);
+            f3 s0 = mk3(0, 0, 0), sx = mk3(0, 0, 0), sy1 = mk3(0, 0, 0);
+            #pragma unroll WHOLLY
+            for (int sy = 0; sy < 3; ++sy) {
+                const bool oy = by + sy >= 4;
+                const uint32_t A = oy ? a1 : a0, B = oy ? b1 : b0, at = lz + 4u * ((by + sy) & 3);
+                const uint32_t ra = A * NODES_PER_BLOCK + at, rb = B * NODES_PER_BLOCK + at;
+                f3 v0, v1, v2;
+                if (WHOLE) {
+                    v0 = node(ra + lx0);
+                    v1 = node((x1 ? rb : ra) + lx1);
+                    v2 = node((x2 ? rb : ra) + lx2);
+                } else {
+                    v0 = A == NONE ? mk3(0, 0, 0) : node(ra + lx0);
+                    v1 = (x1 ? B : A) == NONE ? mk3(0, 0, 0) : node((x1 ? rb : ra) + lx1);
+                    v2 = (x2 ? B : A) == NONE ? mk3(0, 0, 0) : node((x2 ? rb : ra) + lx2);
+                }
+                const f3 c1 = v1 * wx[1], c2 = v2 * wx[2];
+                const f3 r0 = v0 * wx[0] + c1 + c2, rx = c1 + c2 * 2.0f;
+                const float wys = pick(wy, sy);
+                const f3 t0 = r0 * wys;
+                s0 = s0 + t0;
+                sx = sx + rx * wys;
+                sy1 = sy1 + t0 * (float)sy;
+            }
+            const float wzs = pick(wz, sz);
+            const f3 u0 = s0 * wzs;
+            vel = vel + u0;
+            gx = gx + sx * wzs;
+            gy = gy + sy1 * wzs;
+            gz = gz + u0 * (float)sz;
+        }
+    }
+    __device__ __forceinline__ f3 node(uint32_t i) const
+    {
         const float4 g = gridv[i];
-        return none ? mk3(0, 0, 0) : mk3(g.x, g.y, g.z);
+        return mk3(g.x, g.y, g.z);
     }
 };
 
@@ -1543,17 +1596,7 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
                         gz = gz + cw * (float)sz;
                     }
                 } else {
-                    #pragma unroll
-                    for (int q = 0; q < 27; ++q) {
-                        const int sx = NBH[q][0], sy = NBH[q][1], sz = NBH[q][2];
-                        const f3 cv = gather.at(bx + sx, by + sy, bz + sz);
-                        const float wgt = wx[sx] * wy[sy] * wz[sz];
-                        const f3 cw = cv * wgt;
-                        vel = vel + cw;
-                        if (sx == 1) gx = gx + cw; else if (sx == 2) gx = gx + cw * 2.0f;
-                        if (sy == 1) gy = gy + cw; else if (sy == 2) gy = gy + cw * 2.0f;
-                        if (sz == 1) gz = gz + cw; else if (sz == 2) gz = gz + cw * 2.0f;
-                    }
+                    gather.transfer(bx, by, bz, wx, wy, wz, vel, gx, gy, gz);
                 }
                 gradv.c0 = (vel * ref.x + gx * h) * inv_d;
                 gradv.c1 = (vel * ref.y + gy * h) * inv_d;
@@ -1586,7 +1629,7 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
                 const float corrected = fmaxf(psd, -0.3f * h);
                 vel = vel + pn * (dt * -corrected * 1.0e3f);
             }
-            m3 tau;
+            m3 tau = mzero();
             if (tag != 4u) {
                 F = F + mul(gradv * dt, F);
             } else {
@@ -1597,32 +1640,26 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
                 nd = nd < 0.5f ? 0.5f : (nd > 2.0f ? 2.0f : nd);
                 F = m3{{nd, 0, 0}, {0, nd, 0}, {0, 0, nd}};
             }
-            switch (tag) {
-            case 0u: {
-                m3 U, V;
-                f3 sv;
-                svd3(F, U, sv, V);
-                tau = linear_stress_svd(cls.w[0], cls.w[1], U, sv);
-                break;
-            }
-            case 1u: tau = nh_stress(cls.w[0], cls.w[1], F); break;
-            case 2u:
-            case 3u: {
-                m3 U, V;
-                f3 sv;
-                dp_project(cls.w + 3, ps0, ps1, ps2, F, U, sv, V);
-                tau = tag == 2u ? linear_stress_svd(cls.w[10], cls.w[11], U, sv) : nh_stress(cls.w[10], cls.w[11], F);
-                break;
-            }
-            case 4u: tau = fluid_stress(cls.w, F, gradv); break;
-            case 5u: {
+            if (tag == 1u) {
+                tau = nh_stress(cls.w[0], cls.w[1], F);
+            } else if (tag == 4u) {
+                tau = fluid_stress(cls.w, F, gradv);
+            } else if (tag == 5u) {
                 m3 U, V;
                 f3 sv;
                 const float hard = snow_project(cls.w + 1, ps0, F, U, sv, V);
                 tau = linear_stress_svd(cls.w[4] * hard, cls.w[5] * hard, U, sv);
-                break;
-            }
-            default: tau = mzero(); break;
+            } else if (tag <= 3u) {
+                // Corotated linear, and Drucker-Prager over either backbone: one copy of the SVD.
+                m3 U;
+                f3 sv;
+                svd3_us(F, U, sv);
+                const float *lame = cls.w;
+                if (tag != 0u) {
+                    dp_project(cls.w + 3, ps0, ps1, ps2, F, U, sv);
+                    lame += 10;
+                }
+                tau = tag == 3u ? nh_stress(lame[0], lame[1], F) : linear_stress_svd(lame[0], lame[1], U, sv);
             }
             C = gradv * mass - tau * (vol0 * inv_d * dt);
             const bool nan_pos = npos.x != npos.x || npos.y != npos.y || npos.z != npos.z;
