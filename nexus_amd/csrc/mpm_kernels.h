@@ -160,7 +160,8 @@ struct NoallocParticles {
     uint32_t *flags;                               // n: bit 0 enabled, bit 1 fixed, bits 2..15 material
     uint32_t *errors;                              // 1 word (may be null): the substep's error bits
 };
-// Writes the tables, the counters and the input arena (from the caller's arrays).
+// Writes the tables, the counters, the input arena (from the caller's arrays) and its keys:
+// launch_substep follows without its key pass.
 void launch_noalloc_setup(const WorldDev &w, const NoallocTables &t, const NoallocParticles &p, int cap, hipStream_t st);
 // Copies the output arena back to the caller's arrays by particle id.
 void launch_noalloc_unpack(const WorldDev &w, const NoallocParticles &p, uint32_t n, int cap, hipStream_t st);
