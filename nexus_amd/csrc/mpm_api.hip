@@ -1270,7 +1270,7 @@ class World {
         WorldDev w{};
         w.in = arena(cur_);
         w.out = arena(cur_ ^ 1);
-        w.pkey = pkey_.p; w.pdense = pdense_.p; w.prank = prank_.p; w.perm = perm_.p; w.sblock = sblock_.p;
+        w.pslot = pslot_.p; w.pdense = pdense_.p; w.prank = prank_.p; w.perm = perm_.p; w.sblock = sblock_.p;
         w.bscene = bscene_.p; w.bvid = bvid_.p; w.bnp = bnp_.p; w.bfirst = bfirst_.p;
         w.bup = bup_.p; w.bdn = bdn_.p; w.stage = stage_.p; w.gridv = gridv_.p;
         w.hkeys = hkeys_.p; w.hvals = hvals_.p; w.hmark = hmark_.p; w.bprim = bprim_.p; w.bmask = bmask_.p;
@@ -1309,7 +1309,7 @@ class World {
         }
         p_cap_ = cap;
         ++gen_;
-        HIP_TRY(pkey_.reserve(cap));
+        HIP_TRY(pslot_.reserve(cap));
         HIP_TRY(pdense_.reserve(cap));
         HIP_TRY(prank_.reserve(cap));
         HIP_TRY(perm_.reserve(cap));
@@ -1410,7 +1410,7 @@ class World {
         (void)b;
         // Buffers a step in flight may still use are reallocated only after it finished;
         // otherwise the new tables are copied behind it on the stream.
-        // One look-back word per scan tile (k_scan), for each of the two scans.
+        // One look-back word per scan tile (k_scan_slots, k_scan_counts), for each of the two scans.
         const uint32_t scan_stride = (hsum + SCAN_TILE - 1u) / SCAN_TILE + 2u;
         const uint32_t nreg = (uint32_t)region_start.size();
         const bool grow = std::max<size_t>(slots_.size(), 1) > scenes_.n || std::max<size_t>(slots_.size(), 1) > ctr_.n ||
@@ -1807,7 +1807,7 @@ class World {
     uint32_t order_age_ = 0;           // substeps since the particles were last ordered by cell
     size_t ctr_zeroed_ = 0;
     DevBuf<float> arenas_[2];
-    DevBuf<uint32_t> pkey_, pdense_, prank_, perm_, sblock_;
+    DevBuf<uint32_t> pslot_, pdense_, prank_, perm_, sblock_;
     DevBuf<uint32_t> bscene_, bprim_, bmask_, bnp_, bfirst_, bup_, bdn_, hkeys_, hvals_, hmark_;
     DevBuf<SceneClock> clock_;       // per slot
     bool any_adaptive_ = false;
@@ -2677,7 +2677,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     Carver c;
     const size_t o_arena0 = c.take<float>((size_t)NUM_PLANES * p_cap);
     const size_t o_arena1 = c.take<float>((size_t)NUM_PLANES * p_cap);
-    const size_t o_pkey = c.take<uint32_t>(p_cap), o_pdense = c.take<uint32_t>(p_cap), o_prank = c.take<uint32_t>(p_cap);
+    const size_t o_pslot = c.take<uint32_t>(p_cap), o_pdense = c.take<uint32_t>(p_cap), o_prank = c.take<uint32_t>(p_cap);
     const size_t o_perm = c.take<uint32_t>(p_cap), o_sblock = c.take<uint32_t>(p_cap);
     const size_t o_bscene = c.take<uint32_t>(b_total), o_bvid = c.take<int4>(b_total), o_bnp = c.take<uint32_t>(b_total);
     const size_t o_bfirst = c.take<uint32_t>(b_total), o_bup = c.take<uint32_t>(8 * (size_t)b_total);
@@ -2701,7 +2701,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     WorldDev w{};
     w.in = Arena{static_cast<float4 *>(at(o_arena0)), p_cap};
     w.out = Arena{static_cast<float4 *>(at(o_arena1)), p_cap};
-    w.pkey = static_cast<uint32_t *>(at(o_pkey)); w.pdense = static_cast<uint32_t *>(at(o_pdense));
+    w.pslot = static_cast<uint32_t *>(at(o_pslot)); w.pdense = static_cast<uint32_t *>(at(o_pdense));
     w.prank = static_cast<uint32_t *>(at(o_prank)); w.perm = static_cast<uint32_t *>(at(o_perm));
     w.sblock = static_cast<uint32_t *>(at(o_sblock));
     w.bscene = static_cast<uint32_t *>(at(o_bscene)); w.bvid = static_cast<int4 *>(at(o_bvid));

@@ -9,7 +9,7 @@ namespace nxm {
 
 struct WorldDev {
     Arena in, out;                 // particle arenas: read (previous order), written (sorted order)
-    uint32_t *pkey;                // per input slot: packed block key
+    uint32_t *pslot;               // per input slot: its block's hash slot (NONE: no block)
     uint32_t *pdense;              // per input slot: its scene, then (counted) its dense block id or NONE
     uint32_t *prank;               // per input slot: its bound codes, then (counted) its rank inside its block
     uint32_t *perm;                // per sorted position: input slot
