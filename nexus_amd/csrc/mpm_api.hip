@@ -2758,6 +2758,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     // and 79 us, 8000 86 and 91, 16,000 97 and 99, 32,000 103 and 102; P2G at 31,337 mixed 26
     // and 15 us, at 120,001 30 and 18.
     lc.order = n >= 16384u;
+    lc.unsorted = true;
     launch_noalloc_setup(w, t, dp, lc.persistent_blocks, st);
     launch_substep(w, lc, st, nullptr, false);
     launch_noalloc_unpack(w, dp, n, lc.persistent_blocks, st);

@@ -80,6 +80,7 @@ struct LaunchConfig {
     uint64_t p_hint;               // upper bound of particles (grid sizing only)
     int persistent_blocks;         // cap on workgroups of grid-stride kernels
     int p2g_blocks;                // workgroups of the P2G kernel (p2g_workgroups)
+    bool unsorted = false;         // the particles come in the caller's order (with keys: always taken so)
     bool order = false;            // also order the particles inside their blocks by cell (k_cell_order)
     // CPIC worlds: a second stream (default priority) on which the contact particles' G2P
     // runs beside the plain particles' one, forked and joined with these two events.

@@ -762,52 +762,115 @@ __device__ inline void block_info_part(const WorldDev &w, uint32_t group, uint32
     }
 }
 
+// Particles of input slot i's block counted: its block id (d, written to pdense[i]) and the
+// maxima of its run's bound codes.
+struct CountRun {
+    uint32_t d, codes, length, offset;   // codes, length: at the run's head
+    bool valid, head;
+    int first;                           // lane of the head
+};
+__device__ inline CountRun count_run(const WorldDev &w, uint32_t i, uint32_t n)
+{
+    const uint32_t l = lane_id();
+    CountRun r;
+    r.valid = i < n;
+    r.d = NONE;
+    r.codes = 0u;
+    if (r.valid) {
+        const uint32_t s = w.pdense[i];
+        const SceneDev &sc = w.scenes[s];
+        // (Words of a scene that has left may be of an older table: looked up in bounds.)
+        const uint32_t at = w.pslot[i];
+        if (at < w.h_total) r.d = w.hvals[at];
+        r.codes = w.prank[i];
+        r.valid = sc.active != 0u;
+        if (!r.valid) {
+            r.d = NONE;
+        } else if (r.d == NONE) {
+            r.d = w.hvals[sc.h_base + sc.h_cap];   // the overflow block: P2G does not take it
+            r.codes = 0u;
+        }
+        w.pdense[i] = r.d;   // NONE: of a scene that has left
+    }
+    const uint32_t pd = __shfl_up(r.d, 1, WAVE);
+    const bool pv = __shfl_up((int)r.valid, 1, WAVE) != 0;
+    r.head = !r.valid || l == 0 || !pv || pd != r.d;
+    const uint64_t heads = __ballot(r.head);
+    const uint32_t h = run_head(heads, l), end = run_end(heads, h);
+    // The run's maxima of the two code halves, at its head.
+    for (uint32_t o = 1; o < WAVE; o <<= 1) {
+        const uint32_t u = __shfl_down(r.codes, o, WAVE);
+        if (l + o < end) r.codes = max(r.codes & 0xFFFFu, u & 0xFFFFu) | (max(r.codes >> 16, u >> 16) << 16);
+    }
+    r.head = r.head && r.valid;
+    r.length = end - l;
+    r.offset = l - h;
+    r.first = (int)h;
+    return r;
+}
+
+// Particles in the order of the last substep's blocks: an atomic per run.
 __device__ inline void count_part(const WorldDev &w, uint32_t group, uint32_t groups)
 {
     const uint32_t n = w.g->p_in;
     const uint32_t nr = (n + WAVE - 1) / WAVE * WAVE;
-    const uint32_t l = lane_id();
     for (uint32_t i = group * blockDim.x + threadIdx.x; i < nr; i += groups * blockDim.x) {
-        bool valid = i < n;
-        uint32_t d = NONE, codes = 0u;
-        if (valid) {
-            const uint32_t s = w.pdense[i];
-            const SceneDev &sc = w.scenes[s];
-            // (Words of a scene that has left may be of an older table: looked up in bounds.)
-            const uint32_t at = w.pslot[i];
-            if (at < w.h_total) d = w.hvals[at];
-            codes = w.prank[i];
-            valid = sc.active != 0u;
-            if (!valid) d = NONE;
-            else {
-                if (d == NONE) {
-                    d = w.hvals[sc.h_base + sc.h_cap];   // the overflow block: P2G does not take it
-                    codes = 0u;
-                }
-            }
-            w.pdense[i] = d;   // NONE: of a scene that has left
-        }
-        uint32_t pd = __shfl_up(d, 1, WAVE);
-        bool pv = __shfl_up((int)valid, 1, WAVE) != 0;
-        bool head = !valid || l == 0 || !pv || pd != d;
-        uint64_t heads = __ballot(head);
-        uint32_t h = run_head(heads, l);
+        const CountRun r = count_run(w, i, n);
         uint32_t base = 0;
-        const uint32_t end = run_end(heads, h);
-        // The run's maxima of the two code halves, at its head.
-        for (uint32_t o = 1; o < WAVE; o <<= 1) {
-            const uint32_t u = __shfl_down(codes, o, WAVE);
-            if (l + o < end) codes = max(codes & 0xFFFFu, u & 0xFFFFu) | (max(codes >> 16, u >> 16) << 16);
-        }
-        if (head && valid) {
-            base = atomicAdd(&w.bnp[d], end - l);
-            if (codes) {
-                atomicMax((uint32_t *)&w.bvid[d].w, codes & 0xFFFFu);
-                atomicMax(&w.bprim[d], codes >> 16);
+        if (r.head) {
+            base = atomicAdd(&w.bnp[r.d], r.length);
+            if (r.codes) {
+                atomicMax((uint32_t *)&w.bvid[r.d].w, r.codes & 0xFFFFu);
+                atomicMax(&w.bprim[r.d], r.codes >> 16);
             }
         }
-        base = __shfl(base, (int)h, WAVE);
-        if (valid) w.prank[i] = base + (l - h);
+        base = __shfl(base, r.first, WAVE);
+        if (r.valid) w.prank[i] = base + r.offset;
+    }
+}
+
+// Particles in the order the host or a caller has them: a block comes back in many runs, so a
+// workgroup first adds up its runs by block in LDS (120,001 particles line by line, the kernel
+// 23.5 -> 10.7 us; 31,337 of four materials 11 -> 7).
+struct CountSet {
+    static constexpr uint32_t SIZE = 2 * KEY_GROUP;
+    uint32_t block[SIZE], count[SIZE], codes[SIZE], mass_codes[SIZE];
+};
+__device__ inline void count_part_unsorted(const WorldDev &w, CountSet &set, uint32_t group, uint32_t groups)
+{
+    const uint32_t n = w.g->p_in;
+    for (uint32_t c = group * KEY_GROUP; c < n; c += groups * KEY_GROUP) {
+        for (uint32_t k = threadIdx.x; k < CountSet::SIZE; k += KEY_GROUP) {
+            set.block[k] = NONE;
+            set.count[k] = set.codes[k] = set.mass_codes[k] = 0u;
+        }
+        __syncthreads();
+        const uint32_t i = c + threadIdx.x;
+        const CountRun r = count_run(w, i, n);
+        uint32_t at = 0u, base = 0u;
+        if (r.head) {
+            at = r.d * 0x9E3779B9u >> 22;
+            for (;; at = (at + 1u) % CountSet::SIZE) {   // ends: at most half the places are taken
+                const uint32_t prev = atomicCAS(&set.block[at], NONE, r.d);
+                if (prev == NONE || prev == r.d) break;
+            }
+            base = atomicAdd(&set.count[at], r.length);
+            atomicMax(&set.codes[at], r.codes & 0xFFFFu);
+            atomicMax(&set.mass_codes[at], r.codes >> 16);
+        }
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < CountSet::SIZE; k += KEY_GROUP) {
+            const uint32_t d = set.block[k];
+            if (d == NONE) continue;
+            if (set.codes[k]) atomicMax((uint32_t *)&w.bvid[d].w, set.codes[k]);
+            if (set.mass_codes[k]) atomicMax(&w.bprim[d], set.mass_codes[k]);
+            set.count[k] = atomicAdd(&w.bnp[d], set.count[k]);
+        }
+        __syncthreads();
+        if (r.head) base += set.count[at];
+        base = __shfl(base, r.first, WAVE);
+        if (r.valid) w.prank[i] = base + r.offset;
+        __syncthreads();
     }
 }
 
@@ -816,10 +879,17 @@ __device__ inline void count_part(const WorldDev &w, uint32_t group, uint32_t gr
 // chains of dependent reads add up).  The keys carry their hash slots, so a particle's block
 // id is one read.  In sequence and with a hash search per particle: 50,000 particles 7.4 us,
 // now 5.0; 32 scenes 22 and 19; the CPIC sand 8.9 and 6.8.
-__global__ void __launch_bounds__(256) k_block_count(WorldDev w, uint32_t count_groups)
+template <bool UNSORTED>
+__global__ void __launch_bounds__(UNSORTED ? KEY_GROUP : 256) k_block_count(WorldDev w, uint32_t count_groups)
 {
-    if (blockIdx.x < count_groups) count_part(w, blockIdx.x, count_groups);
-    else block_info_part(w, blockIdx.x - count_groups, gridDim.x - count_groups);
+    if (blockIdx.x >= count_groups) {
+        block_info_part(w, blockIdx.x - count_groups, gridDim.x - count_groups);
+    } else if constexpr (UNSORTED) {
+        __shared__ CountSet set;
+        count_part_unsorted(w, set, blockIdx.x, count_groups);
+    } else {
+        count_part(w, blockIdx.x, count_groups);
+    }
 }
 
 // P2G work split: workgroup g of the P2G grid takes blocks [p2g_start[g], p2g_start[g+1]),
@@ -2547,6 +2617,11 @@ static inline int g2p_groups(uint64_t p_hint, int threads)
 // (2^17 slots), 10.8 and 15.3 for 32 scenes, 80 and 23 at 2^22 slots.
 constexpr uint32_t SMALL_HASH = 1u << 20;
 
+// Particles from which an unsorted count goes through LDS: few particles have few runs per
+// block, and its barriers show.  Calls without and with: 5000 of one material 69-70 and
+// 71-72 us, 8000 75-77 and 74-77 (sand 78 and 73), 12,000 80-82 and 75-78, 32,000 sand 91 and 87.
+constexpr uint64_t UNSORTED_MIN = 8192;
+
 void launch_substep(const WorldDev &w, const LaunchConfig &lc, hipStream_t st, hipEvent_t *ev, bool keys)
 {
     const int T = 256;
@@ -2564,8 +2639,12 @@ void launch_substep(const WorldDev &w, const LaunchConfig &lc, hipStream_t st, h
     };
     if (w.h_total <= SMALL_HASH) slots(k_scan_slots<4, 4>, 4 * WAVE, slot_tile<4, 4>());
     else slots(k_scan_slots<16, 16>, 16 * WAVE, slot_tile<16, 16>());
-    const int counting = grid_for(lc.p_hint, T, cap);
-    k_block_count<<<counting + grid_for((uint64_t)w.b_total * 16, T, cap), T, 0, st>>>(w, (uint32_t)counting);
+    auto count = [&](auto kernel, int threads) {
+        const int counting = grid_for(lc.p_hint, threads, cap);
+        kernel<<<counting + grid_for((uint64_t)w.b_total * 16, threads, cap), threads, 0, st>>>(w, (uint32_t)counting);
+    };
+    if ((keys || lc.unsorted) && lc.p_hint >= UNSORTED_MIN) count(k_block_count<true>, KEY_GROUP);
+    else count(k_block_count<false>, T);
     const uint32_t btile = SCAN_TILE * scan_chunks(w.b_total);
     const int bscan = std::min((int)((w.b_total + btile - 1) / btile), cap);
     k_scan_counts<<<std::max(bscan, 1), 256, 0, st>>>(w);

@@ -26,7 +26,7 @@ def _scene(n, per_block, seed):
 
 
 @pytest.mark.parametrize("n,per_block", [(1, 1), (64, 1), (65, 2), (511, 1), (512, 1), (513, 3), (1025, 1), (4096, 1),
-                                         (6001, 64), (16383, 40), (16384, 40)])
+                                         (6001, 64), (8191, 40), (8192, 40), (16383, 40), (16384, 40)])
 def test_key_pass(pipeline, n, per_block):
     sc = _scene(n, per_block, 0)
     cap = 32768
