@@ -2,8 +2,8 @@
 //
 // One substep over every active scene of a world (device data in WorldDev):
 //   k_clear         clear hash regions, block tables and counters, then
-//   k_keys_touch    per particle: block key; per run of equal keys in a wave, insertion
-//                   of the block and its 7 +1 neighbours (both only for the first substep
+//   k_keys_touch    per particle: block key; per block that a workgroup meets, insertion
+//                   of it and its 7 +1 neighbours (both only for the first substep
 //                   and after the host changed the arena or the tables: otherwise the
 //                   previous substep's k_g2p_update made the keys and insertions)
 //   k_scan_slots    single-pass scan of occupied hash slots -> dense block ids
@@ -11,6 +11,7 @@
 //                   per particle: dense block id, wave-aggregated block counts and ranks
 //   k_scan_counts   single-pass scan of block counts -> first particle of each block
 //   k_scatter       per particle: sorted position (block-major permutation)
+//   k_cell_order    now and then: the order of the particles inside their blocks
 //   k_p2g           per block: LDS-staged scatter of its particles into a 6^3 node tile
 //   k_grid_update   per node: sum of the tiles covering it, momentum -> velocity, gravity,
 //                   clamp, cuboid colliders; empties the hash
