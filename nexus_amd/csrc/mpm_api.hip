@@ -86,27 +86,29 @@ using namespace nxm;
 
 // Pinned host chunks shared by the threads of one context: a scene staged for upload on
 // one thread (nxm_scene_stage_upload) holds a chunk until the thread stepping its world
-// queues the copies; the chunk is reused once those copies have executed.
+// queues the copies; the chunk is reused once those copies have executed.  Readbacks have
+// chunks of their own, given back when nothing is queued on them: they need no event, and so
+// never ask for one last recorded on a stream that has gone or is being captured.
 struct PinnedPool {
     struct Chunk {
         char *p = nullptr;
         size_t n = 0;
-        hipEvent_t ev = nullptr;
+        hipEvent_t ev = nullptr;   // null: a readback's
         bool held = false;
     };
     std::mutex mu;
     std::vector<Chunk> chunks;
 
     // The smallest free chunk of at least `bytes` whose last copies have executed.
-    hipError_t take(size_t bytes, int *idx, char **out)
+    hipError_t take(size_t bytes, int *idx, char **out, bool readback = false)
     {
         std::lock_guard<std::mutex> g(mu);
         int best = -1;
         for (int k = 0; k < (int)chunks.size(); ++k) {
             Chunk &c = chunks[k];
-            if (c.held || c.n < bytes) continue;
+            if (c.held || c.n < bytes || readback != (c.ev == nullptr)) continue;
             if (best >= 0 && chunks[best].n <= c.n) continue;
-            const hipError_t q = hipEventQuery(c.ev);
+            const hipError_t q = readback ? hipSuccess : hipEventQuery(c.ev);
             if (q == hipErrorNotReady) continue;
             if (q != hipSuccess) return q;
             best = k;
@@ -116,7 +118,7 @@ struct PinnedPool {
             c.n = std::max<size_t>(bytes, (size_t)1 << 20);
             hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&c.p), c.n, hipHostMallocDefault);
             if (e != hipSuccess) return e;
-            e = hipEventCreate(&c.ev);
+            if (!readback) e = hipEventCreate(&c.ev);
             if (e != hipSuccess) { (void)hipHostFree(c.p); return e; }
             chunks.push_back(c);
             best = (int)chunks.size() - 1;
@@ -143,8 +145,10 @@ struct PinnedPool {
     ~PinnedPool()
     {
         for (auto &c : chunks) {
-            (void)hipEventSynchronize(c.ev);
-            (void)hipEventDestroy(c.ev);
+            if (c.ev) {
+                (void)hipEventSynchronize(c.ev);
+                (void)hipEventDestroy(c.ev);
+            }
             (void)hipHostFree(c.p);
         }
     }
@@ -800,7 +804,7 @@ class World {
         const size_t nslots = std::min(slots_.size(), ctr_.n);
         int held = -1;
         char *pin = nullptr;
-        HIP_TRY(ctx_->pool.take(2 * READ_CHUNK + MAX_SCENES * sizeof(SceneCtr), &held, &pin));
+        HIP_TRY(ctx_->pool.take(2 * READ_CHUNK + MAX_SCENES * sizeof(SceneCtr), &held, &pin, true));
         nxm_status st = copy_through(pin, reinterpret_cast<const char *>(dev), total, parts, nslots);
         if (st != NXM_OK) (void)hipStreamSynchronize(stream_);   // nothing still writes the chunk
         HIP_TRY(ctx_->pool.give(held, nullptr));
