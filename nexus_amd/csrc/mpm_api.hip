@@ -569,12 +569,6 @@ class World {
             for (auto &e : ring_) (void)hipEventDestroy(e);
             for (auto &e : read_ev_)
                 if (e) (void)hipEventDestroy(e);
-            if (side_) {
-                (void)hipStreamSynchronize(side_);
-                (void)hipEventDestroy(fork_);
-                (void)hipEventDestroy(join_);
-                (void)hipStreamDestroy(side_);
-            }
             (void)hipStreamDestroy(stream_);
         }
     }
@@ -906,9 +900,6 @@ class World {
         lc.p_hint = p_in_;
         lc.persistent_blocks = (int)cfg.grid_groups;
         lc.p2g_blocks = (int)w.p2g_groups;
-        lc.side = side_;
-        lc.fork = fork_;
-        lc.join = join_;
         hipEvent_t *evs = times ? ev_ : nullptr;
         if (!times && profiling_ && profile_seen_++ % profile_every_ == 0) {
             nxm_status st = ring_events(&evs);
@@ -1522,13 +1513,6 @@ class World {
             HIP_TRY(gridv_i_.reserve((size_t)NODES_PER_BLOCK * nb));
         }
         any_cpic_ = any_cpic;
-        if (any_cpic && !side_) {
-            // Created with the first CPIC scene only: streams are spread over the device's
-            // hardware queues in creation order, and worlds without CPIC keep one stream each.
-            HIP_TRY(hipStreamCreateWithFlags(&side_, hipStreamNonBlocking));
-            HIP_TRY(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
-            HIP_TRY(hipEventCreateWithFlags(&join_, hipEventDisableTiming));
-        }
         if (any_mesh) {
             // k_grid_cdf empties every node k_mesh_cdf wrote in the same substep; fresh
             // allocations are emptied here, outside any captured graph.
@@ -1779,8 +1763,6 @@ class World {
 
     nxm_ctx *ctx_;
     hipStream_t stream_ = nullptr;
-    hipStream_t side_ = nullptr;       // CPIC: the contact particles' G2P (default priority)
-    hipEvent_t fork_ = nullptr, join_ = nullptr;
     nxm_launch_config cfg_{};
     bool tune_on_ = false, tuning_ = false;
     int tune_stage_ = 0, tune_rep_ = 0;

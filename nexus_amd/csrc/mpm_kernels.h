@@ -82,10 +82,6 @@ struct LaunchConfig {
     int p2g_blocks;                // workgroups of the P2G kernel (p2g_workgroups)
     bool unsorted = false;         // the particles come in the caller's order (with keys: always taken so)
     bool order = false;            // also order the particles inside their blocks by cell (k_cell_order)
-    // CPIC worlds: a second stream (default priority) on which the contact particles' G2P
-    // runs beside the plain particles' one, forked and joined with these two events.
-    hipStream_t side = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
 };
 
 // Substeps between two orderings of the particles inside their blocks (LaunchConfig::order).

@@ -19,7 +19,7 @@
 //                   written in sorted order to the output arena; then the next substep's
 //                   block keys and insertions
 // CPIC worlds add the contact fields (k_mesh_cdf, k_grid_cdf, k_particle_cdf) before P2G,
-// the CPIC variants of the transfers, k_g2p_contact and k_integrate_colliders.
+// the CPIC variants of the transfers, and k_g2p_contact before k_g2p_update.
 // The reference runs the same stages as ~21 dispatches (src_mpm/pipeline.rs:385-526).
 #include <type_traits>
 
@@ -59,8 +59,8 @@ constexpr uint32_t NUM_XCD = 8;
 
 // Workgroup size of k_g2p_update (one particle per thread): two waves, measured fastest for
 // the plain kernel (256: sand column G2P 1 us, clumped fluid 5-7 % slower; 192: the fluid 6 %
-// slower; 64 and 512 slower too); CPIC worlds keep 256, which shares the GPU better with the contact G2P running
-// beside it (128: CPIC sand column 4 % slower).
+// slower; 64 and 512 slower too); CPIC worlds keep 256 (128: the
+// same from 60,000 to 1M particles, 2 % faster at 262,144).
 template <bool CPIC> constexpr int g2p_threads() { return CPIC ? 256 : 128; }
 
 __device__ inline void xcd_range(uint32_t n, uint32_t &begin, uint32_t &end)
@@ -2071,8 +2071,6 @@ __device__ inline void integrate_colliders_part(const WorldDev &w)
     }
 }
 
-__global__ void __launch_bounds__(256) k_integrate_colliders(WorldDev w) { integrate_colliders_part(w); }
-
 // Contact particles of CPIC scenes: those with affinity bits (the others are compatible
 // with every node and have a zero contact field, so the plain path is exact for them).
 __device__ inline bool contact_particle(const WorldDev &w, uint32_t pos, uint32_t d)
@@ -2241,7 +2239,7 @@ __global__ void __launch_bounds__(g2p_threads<CPIC>()) k_g2p_update(WorldDev w)
         if (ADAPT) next_dt_bound(w, pos, valid, s);
     }
     prepare_next_sort(w);
-    if (!CPIC) integrate_colliders_part(w);   // CPIC worlds: after k_g2p_contact, which reads them
+    integrate_colliders_part(w);   // their last reader (k_g2p_contact, in CPIC worlds) has run
 }
 
 // The contact particles listed by k_particle_cdf, then their keys (as in k_g2p_update).
@@ -2666,26 +2664,17 @@ void launch_substep(const WorldDev &w, const LaunchConfig &lc, hipStream_t st, h
         if (w.mesh_pass) k_grid_update<true, true><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
         else k_grid_update<true, false><<<grid_for((uint64_t)w.b_total * 64, T, cap), T, 0, st>>>(w);
         if (ev) (void)hipEventRecord(ev[3], st);
-        // The contact particles' G2P touches other particles than the plain one and is
-        // latency-bound on few waves: it runs beside it on the side stream when there is one.
-        hipStream_t cs = st;
-        if (lc.side && lc.fork && lc.join) {
-            (void)hipEventRecord(lc.fork, st);
-            (void)hipStreamWaitEvent(lc.side, lc.fork, 0);
-            cs = lc.side;
-        }
+        // The contact particles' G2P, then the plain particles', which also integrates the
+        // bodies.  (Side by side on two streams the fork, the join and a launch for the bodies
+        // cost more than the overlap gave, frames of 20 substeps: 60,000 particles 2925 -> 2618
+        // us, 262,144 3875 -> 3600, 1,048,576 7865 -> 7650, sand on a mesh ramp 3350 -> 3127.)
         // Adaptive worlds take the variants that also min-reduce the next substep's bound.
-        if (w.any_adaptive) k_g2p_contact<true><<<grid_for(lc.p_hint, T, cap), T, 0, cs>>>(w);
-        else k_g2p_contact<false><<<grid_for(lc.p_hint, T, cap), T, 0, cs>>>(w);
+        if (w.any_adaptive) k_g2p_contact<true><<<grid_for(lc.p_hint, T, cap), T, 0, st>>>(w);
+        else k_g2p_contact<false><<<grid_for(lc.p_hint, T, cap), T, 0, st>>>(w);
         auto g2p = w.any_adaptive ? k_g2p_update<true, true> : k_g2p_update<true, false>;
         constexpr int GT = g2p_threads<true>();
         if (ev) hipExtLaunchKernelGGL(g2p, dim3(g2p_groups(lc.p_hint, GT)), dim3(GT), 0, st, ev[7], ev[8], 0, w);
         else g2p<<<g2p_groups(lc.p_hint, GT), GT, 0, st>>>(w);
-        if (cs != st) {
-            (void)hipEventRecord(lc.join, cs);
-            (void)hipStreamWaitEvent(st, lc.join, 0);
-        }
-        k_integrate_colliders<<<std::max(1, (int)((w.s_count * 16u + T - 1) / T)), T, 0, st>>>(w);
     } else {
         if (ev) hipExtLaunchKernelGGL(k_p2g<false>, dim3(pg), dim3(P2G_WAVES * WAVE), 0, st, ev[5], ev[6], 0, w);
         else k_p2g<false><<<pg, P2G_WAVES * WAVE, 0, st>>>(w);
