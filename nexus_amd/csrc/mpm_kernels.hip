@@ -188,15 +188,15 @@ __device__ inline P2GIn p2g_load(const WorldDev &w, uint32_t slot)
 
 // Bounds of a particle's P2G contributions, |m v + C dpt| (|dpt_j| <= 1.5 h) and m, as the
 // exponents of the powers of two above them: the low half and the high half of one word, 0
-// for none, CODE_HUGE for a bound that is not finite (NaN components are left out, as fmaxf
-// does).  Made where a particle's key is made, from the state still in registers; the
-// count kernel takes a block's maxima, so that P2G reads a block's particles once.
+// for none.  A bound that is not finite counts as none, so that a block's scale is that of
+// its other particles (p2g_one checks every contribution of such a particle); NaN
+// components are left out, as fmaxf does.  Made where a particle's key is made, from the
+// state still in registers; the count kernel takes a block's maxima, so that P2G reads a
+// block's particles once.
 constexpr int CODE_BIAS = 200;
-constexpr uint32_t CODE_HUGE = 511u;
 __device__ inline uint32_t bound_code(float b)
 {
-    if (!(b > 0.0f)) return 0u;
-    if (!isfinite(b)) return CODE_HUGE;
+    if (!(b > 0.0f) || !isfinite(b)) return 0u;
     int e;
     (void)frexpf(b, &e);   // b = m 2^e, m in [0.5, 1): b < 2^e
     return (uint32_t)(e + CODE_BIAS);
@@ -1035,7 +1035,7 @@ struct Fixed {
 // (bound_code).
 __device__ inline float fixed_scale(uint32_t code, uint32_t np)
 {
-    const int e = code < 2u || code >= CODE_HUGE ? 0 : (int)code - CODE_BIAS;
+    const int e = code < 2u ? 0 : (int)code - CODE_BIAS;   // 0, 1: no bound (of a marked block)
     const int lg = np > 1u ? 32 - __clz((int)(np - 1u)) : 0;   // ceil(log2 np)
     int k = Fixed::BITS - e - max(lg - Fixed::FREE_LOG2, 0);
     k = k > 126 ? 126 : (k < -126 ? -126 : k);
@@ -1125,9 +1125,9 @@ __device__ __forceinline__ void p2g_scatter(unsigned long long *tile, const Sten
     }
 }
 
-// The same for a particle that may give contributions that are not finite or beyond the
-// conversion's range: those are marked, and the node reads NaN.  Rare, so one loop over
-// nodes [q0, q1) of the stencil.
+// The same for a particle whose bound is not finite (it is not in the block's): its
+// contributions beyond the conversion's range are marked, and the node reads NaN.  Rare, so
+// one loop over nodes [q0, q1) of the stencil.
 template <int PART>
 __device__ __forceinline__ void p2g_scatter_checked(unsigned long long *tile, uint32_t *bad, const Stencil &q, int q0,
                                                     int q1, const uint32_t *naff, uint32_t pa)
@@ -1273,7 +1273,6 @@ __device__ __forceinline__ void stencil_weights(float f, float (&w)[3])
 struct BlockScales {
     int4 v;
     float h, ih, smom, sm;
-    bool huge;              // a bound beyond 2^100: check every contribution
 };
 __device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t s, int4 v, uint32_t mass_code, uint32_t np)
 {
@@ -1283,7 +1282,6 @@ __device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t 
     b.ih = ld_uniform(&w.scenes[s].inv_h);
     b.smom = fixed_scale((uint32_t)v.w, np);
     b.sm = fixed_scale(mass_code, np);
-    b.huge = (uint32_t)v.w > CODE_BIAS + 100u || mass_code > CODE_BIAS + 100u;
     return b;
 }
 
@@ -1294,14 +1292,15 @@ __device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *
                                             uint32_t sel, const uint32_t *naff, uint32_t pa)
 {
     const float h = b.h, ih = b.ih;
-    // With finite inputs and a finite block bound far below FLT_MAX every contribution is
-    // finite (|contribution| <= bound): only other particles take the checked scatter.
-    float z = p.px * 0.0f;   // NaN if any input is not finite
-    z = __builtin_fmaf(p.py, 0.0f, __builtin_fmaf(p.pz, 0.0f, __builtin_fmaf(p.m, 0.0f, z)));
-    z = __builtin_fmaf(p.v.x, 0.0f, __builtin_fmaf(p.v.y, 0.0f, __builtin_fmaf(p.v.z, 0.0f, z)));
-    z = __builtin_fmaf(p.C.c0.x, 0.0f, __builtin_fmaf(p.C.c0.y, 0.0f, __builtin_fmaf(p.C.c0.z, 0.0f, z)));
-    z = __builtin_fmaf(p.C.c1.x, 0.0f, __builtin_fmaf(p.C.c1.y, 0.0f, __builtin_fmaf(p.C.c1.z, 0.0f, z)));
-    z = __builtin_fmaf(p.C.c2.x, 0.0f, __builtin_fmaf(p.C.c2.y, 0.0f, __builtin_fmaf(p.C.c2.z, 0.0f, z)));
+    // A sum that bounds |m v + C dpt|: finite and far below FLT_MAX, it says that the bound
+    // code did count this particle, so that its contributions fit the block's scale.  Any
+    // other particle (a NaN or an infinity among its inputs, or a bound that overflows) takes
+    // the checked scatter.
+    const float vsum = fabsf(p.v.x) + fabsf(p.v.y) + fabsf(p.v.z);
+    const float csum = fabsf(p.C.c0.x) + fabsf(p.C.c0.y) + fabsf(p.C.c0.z) + fabsf(p.C.c1.x) + fabsf(p.C.c1.y) +
+                       fabsf(p.C.c1.z) + fabsf(p.C.c2.x) + fabsf(p.C.c2.y) + fabsf(p.C.c2.z);
+    float sum = __builtin_fmaf(4.5f * h, csum, fabsf(p.m) * vsum);
+    sum = __builtin_fmaf(p.px, 0.0f, __builtin_fmaf(p.py, 0.0f, __builtin_fmaf(p.pz, 0.0f, sum)));
     // Base node of the stencil and its offset from the particle.
     const float cx = round_div(p.px, h, ih) - 1.0f, cy = round_div(p.py, h, ih) - 1.0f, cz = round_div(p.pz, h, ih) - 1.0f;
     const int bx = (int)cx - 4 * b.v.x, by = (int)cy - 4 * b.v.y, bz = (int)cz - 4 * b.v.z;
@@ -1326,7 +1325,7 @@ __device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *
     q.hy = scaled(p.C.c1, hs);
     q.hz = scaled(p.C.c2, hs);
     q.mass = (double)p.m * (double)b.sm;
-    if (b.huge || !(z == 0.0f)) p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K), naff, pa);
+    if (!(sum < 0x1p120f) || !(fabsf(p.m) < 0x1p120f)) p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K), naff, pa);
     else p2g_scatter<PART, K>(tile, q, (int)sel, naff, pa);
     return spill_mask(bx, by, bz);
 }
