@@ -1003,41 +1003,50 @@ __global__ void __launch_bounds__(WAVE) k_cell_order(WorldDev w)
 //
 // The tile accumulates in 64-bit fixed point with integer LDS atomics (ds_add_u64):
 // float LDS atomics serialize on gfx950 (~200 cycles per wave-op against ~8 for the
-// 64-bit integer add).  A first pass bounds the block's contributions by 2^e; the scale
-// 2^(51 - e) then resolves each contribution to 2^-52 of that bound, and a node's sum stays
-// below 2^62 for up to 2048 particles in the block (above, the scale gives up a bit per
-// doubling).  Integer sums do not depend on the order of the adds, so the tile is
-// bit-reproducible whatever the particle order.
+// 64-bit integer add).  The block's contributions are bounded by 2^e (bound_codes, reduced
+// by the count kernel); a tile node receives at most np of them (one per particle of the
+// block), so the scale 2^(62 - e - ceil(log2 np)) keeps every node sum below 2^62 while
+// resolving contributions down to 2^-62 np of the largest.  Integer sums do not depend on
+// the order of the adds, so the tile is bit-reproducible whatever the particle order.
 
 // 64-bit fixed-point accumulator words of the P2G tile.
 struct Fixed {
     using word = unsigned long long;
-    // Contributions are formed in double and rounded to the tile's unit by adding 1.5 2^52:
-    // for |a w| < 2^51 the sum's mantissa holds round(a w) in two's complement, and its bit
-    // pattern minus that of 1.5 2^52 (whose low word is zero) is the integer: one fused
-    // multiply-add and one 32-bit subtraction per contribution.  Doubles run at the rate of
-    // floats here, so this replaced the multiply and five operations that split a float into
-    // two 32-bit halves.  The product is exact before that one rounding, so an integer
+    // round(a w) as a two's-complement 64-bit integer, |a w| < 2^62: contributions are formed
+    // in double and rounded once.  t = a w + 1.5 2^84 holds the high part H = round(a w / 2^32)
+    // 2^32 in its low mantissa word; with it taken off exactly, r = a w - H + 1.5 2^52, where
+    // |a w - H| <= 2^31, holds the rest in its mantissa.  The pattern of r plus H is the
+    // integer plus that of 1.5 2^52, which ONE takes off (its low word is zero, so that it
+    // can stand in t): three double operations and one 32-bit sum.  Doubles run at
+    // the rate of floats here.  The product is exact before each rounding, so an integer
     // depends on a and w alone.
-    static constexpr int BITS = 51;
-    static constexpr int FREE_LOG2 = 11;        // particles whose sum needs no headroom bits
-    static constexpr double LIMIT = 0x1p51;     // |a w| below this: an exact conversion
+    // One rounding to a unit of 2^(e - 51) takes a third of the double operations (P2G of 1M
+    // sand 78 us against 83, of 2M clumped fluid 400 against 421), but small contributions,
+    // such as the mass at the rim of a stencil, then have up to 11 bits less.
+    static constexpr int BITS = 62;
+    static constexpr double ONE = (double)0x43380000u * 0x1p32, T = 0x1.8p84 - ONE, R = 0x1.8p52;
     __device__ static word of(double a, double w)
     {
-        const unsigned long long t = (unsigned long long)__double_as_longlong(__builtin_fma(a, w, 0x1.8p52));
-        return ((unsigned long long)((uint32_t)(t >> 32) - 0x43380000u) << 32) | (uint32_t)t;
+        const double t = __builtin_fma(a, w, T);
+        const double r = __builtin_fma(a, w, (T + R) - t);   // (T + R and the difference: exact)
+        const uint32_t h = (uint32_t)__double_as_longlong(t);
+        union { double d; uint32_t w[2]; word all; } u{r};
+        // (written out: as plain sums the compiler makes two 64-bit ones of it)
+        asm("v_add_u32 %0, %1, %2" : "=v"(u.w[1]) : "v"(u.w[1]), "v"(h));
+        return u.all;
     }
     // scale is a power of two: multiplying by its reciprocal is exact
     __device__ static float back(word x, double inv_scale) { return (float)((double)(long long)x * inv_scale); }
 };
+
+__device__ inline int log2_up(uint32_t np) { return np > 1u ? 32 - __clz((int)(np - 1u)) : 0; }   // ceil(log2 np)
 
 // The scale of a block whose contributions are bounded by 2^e, from the bound's code
 // (bound_code).
 __device__ inline float fixed_scale(uint32_t code, uint32_t np)
 {
     const int e = code < 2u ? 0 : (int)code - CODE_BIAS;   // 0, 1: no bound (of a marked block)
-    const int lg = np > 1u ? 32 - __clz((int)(np - 1u)) : 0;   // ceil(log2 np)
-    int k = Fixed::BITS - e - max(lg - Fixed::FREE_LOG2, 0);
+    int k = Fixed::BITS - e - log2_up(np);
     k = k > 126 ? 126 : (k < -126 ? -126 : k);
     return ldexpf(1.0f, k);
 }
@@ -1096,8 +1105,8 @@ __device__ __forceinline__ void add_node(unsigned long long *tile, int t, d3 a, 
 // K lanes share one particle: K = 1 scatters all 27 stencil nodes; K = 3 the 9 nodes of z
 // slab sel; K = 9 the 3 nodes of row (sz, sy) = (sel / 3, sel % 3); K = 27 node (sel / 9,
 // sel / 3 % 3, sel % 3).  Every node's contribution is computed by the same operations
-// whatever K is (each step an explicit fused multiply-add, exact for an offset of 0), so
-// which lanes take a particle changes no bit.
+// whatever K is (each step an explicit fused multiply-add; one with an offset of 0 is exact,
+// and left out where the offset is known), so which lanes take a particle changes no bit.
 template <int PART, int K>
 __device__ __forceinline__ void p2g_scatter(unsigned long long *tile, const Stencil &q, int sel, const uint32_t *naff,
                                             uint32_t pa)
@@ -1113,24 +1122,25 @@ __device__ __forceinline__ void p2g_scatter(unsigned long long *tile, const Sten
         #pragma unroll
         for (int ky = 0; ky < NY; ++ky) {
             const int sy = NY == 3 ? ky : (K == 9 ? sel % 3 : (sel / 3) % 3);
-            const d3 ay = step(az, q.hy, (double)sy);
+            const d3 ay = NY == 3 && ky == 0 ? az : step(az, q.hy, (double)sy);   // (a step of 0 adds nothing)
             const double wyz = (double)pick(q.wy, sy) * wzs;
             #pragma unroll
             for (int kx = 0; kx < NX; ++kx) {
                 const int sx = NX == 3 ? kx : sel % 3;
                 const int t = q.t0 + sx + TILE * sy + TILE * TILE * sz;
-                if (adds_to<PART>(naff, t, pa)) add_node(tile, t, step(ay, q.hx, (double)sx), q.mass, (double)pick(q.wx, sx) * wyz);
+                const d3 a = NX == 3 && kx == 0 ? ay : step(ay, q.hx, (double)sx);
+                if (adds_to<PART>(naff, t, pa)) add_node(tile, t, a, q.mass, (double)pick(q.wx, sx) * wyz);
             }
         }
     }
 }
 
 // The same for a particle whose bound is not finite (it is not in the block's): its
-// contributions beyond the conversion's range are marked, and the node reads NaN.  Rare, so
-// one loop over nodes [q0, q1) of the stencil.
+// contributions beyond the others' range (limit, np of which fit a word) are marked, and
+// the node reads NaN.  Rare, so one loop over nodes [q0, q1) of the stencil.
 template <int PART>
 __device__ __forceinline__ void p2g_scatter_checked(unsigned long long *tile, uint32_t *bad, const Stencil &q, int q0,
-                                                    int q1, const uint32_t *naff, uint32_t pa)
+                                                    int q1, double limit, const uint32_t *naff, uint32_t pa)
 {
     #pragma unroll 1
     for (int n = q0; n < q1; ++n) {
@@ -1140,7 +1150,7 @@ __device__ __forceinline__ void p2g_scatter_checked(unsigned long long *tile, ui
         const d3 a = step(step(step(q.base, q.hz, (double)sz), q.hy, (double)sy), q.hx, (double)sx);
         const double wgt = (double)pick(q.wx, sx) * ((double)pick(q.wy, sy) * (double)pick(q.wz, sz));
         add_node(tile, t, a, q.mass, wgt);
-        auto off = [&](double v) { return !(fabs(v * wgt) < Fixed::LIMIT); };   // NaN too
+        auto off = [&](double v) { return !(fabs(v * wgt) < limit); };   // NaN too
         if (off(a.x) || off(a.y) || off(a.z) || off(q.mass)) {
             atomicOr(&bad[BAD_ANY], 1u);
             for (int c = 0; c < TILE_FIELDS; ++c) {
@@ -1273,6 +1283,7 @@ __device__ __forceinline__ void stencil_weights(float f, float (&w)[3])
 struct BlockScales {
     int4 v;
     float h, ih, smom, sm;
+    uint32_t np;
 };
 __device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t s, int4 v, uint32_t mass_code, uint32_t np)
 {
@@ -1282,6 +1293,7 @@ __device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t 
     b.ih = ld_uniform(&w.scenes[s].inv_h);
     b.smom = fixed_scale((uint32_t)v.w, np);
     b.sm = fixed_scale(mass_code, np);
+    b.np = np;
     return b;
 }
 
@@ -1325,8 +1337,11 @@ __device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *
     q.hy = scaled(p.C.c1, hs);
     q.hz = scaled(p.C.c2, hs);
     q.mass = (double)p.m * (double)b.sm;
-    if (!(sum < 0x1p120f) || !(fabsf(p.m) < 0x1p120f)) p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K), naff, pa);
-    else p2g_scatter<PART, K>(tile, q, (int)sel, naff, pa);
+    if (!(sum < 0x1p120f) || !(fabsf(p.m) < 0x1p120f))
+        p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K),
+                                  ldexp(1.0, Fixed::BITS - log2_up(b.np)), naff, pa);
+    else
+        p2g_scatter<PART, K>(tile, q, (int)sel, naff, pa);
     return spill_mask(bx, by, bz);
 }
 

@@ -1,9 +1,10 @@
-"""P2G of blocks in which one particle's contributions cannot be held: they mark the nodes of
-that particle's stencil and no others, whatever the size of the block's other values."""
+"""The range and the resolution of P2G's sums: a particle whose contributions cannot be held
+marks the nodes of its stencil and no others, whatever the size of the block's other values,
+and small contributions keep the bits that the block's unit has for them."""
 import numpy as np
 import pytest
 
-from nexus_amd import mpm
+from nexus_amd import mpm, scenes
 
 from test_gpu_p2g_blocks import _scene
 
@@ -59,3 +60,39 @@ def test_marks_stay_in_the_stencil(pipeline, count, kind):
     for f in ("x", "v", "C", "F"):
         scale = np.abs(a[f]).max()
         assert np.abs(a[f][far] - b[f][far]).max() <= 1e-5 * scale, f
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 7, 21, 22, 64, 65, 129, 1025])
+def test_small_contributions(pipeline, count):
+    """Particles at 2^-4 to 2^-10 of a cell from the rim of their stencils, where the weights
+    (down to 2^-63) are exact: every node's sums against 64 bits, to half the block's unit
+    2^(e + ceil(log2 n) - 62) per particle and the FP32 rounding of the node."""
+    h = 0.25
+    rng = np.random.default_rng(count)
+    cell = rng.integers(0, 4, (count, 3))
+    a = 2.0 ** -rng.choice([4, 6, 8, 10], (count, 3))
+    a[0] = 2.0 ** -10
+    sc = scenes.make_scene(scenes.particles((cell + 1.5 - a) * h, h / 4, 1000.0, scenes.model_neo_hookean(1e5, 0.3),
+                                            velocity=rng.normal(0, 0.5, (count, 3))), h, 1e-3)
+    sc.mass[:] = rng.uniform(0.5, 1.5, count).astype(np.float32)
+    sc.C = rng.normal(0, 2.0, (count, 9)).astype(np.float32)
+    m, v, C = sc.mass.astype(float), sc.v.astype(float), sc.C.astype(float).reshape(-1, 3, 3)   # C[:, j]: column j
+    w = np.stack([0.5 * a * a, 0.75 - (0.5 - a) ** 2, 0.5 * (1 - a) ** 2])                       # [offset, particle, axis]
+    bound = 4.5 * h * np.abs(C).max((1, 2)) + m * np.abs(v).max(1)
+    unit = [2.0 ** (np.frexp(np.float32(b.max() * (1 + 1e-6)))[1] + int(np.ceil(np.log2(count))) - 62) for b in (m, bound)]
+    want, hits = {}, {}
+    for i in range(3):
+        for j in range(3):
+            for k in range(3):
+                wt = w[i, :, 0] * w[j, :, 1] * w[k, :, 2]
+                dpt = (np.array([i, j, k]) - (1.5 - a)) * h
+                mom = (m[:, None] * v + (C * dpt[:, :, None]).sum(1)) * wt[:, None]
+                for p in range(count):
+                    key = tuple((cell[p] + (i, j, k)).tolist())
+                    want[key] = want.get(key, 0.0) + np.array([m[p] * wt[p], *mom[p]])
+                    hits[key] = hits.get(key, 0) + 1
+    got, _ = _run(pipeline, sc)
+    for key, t in want.items():
+        tol = 0.5 * hits[key] * np.array([unit[0], unit[1], unit[1], unit[1]]) + 2.0 ** -23 * np.abs(t)
+        err = np.abs(np.array(got[key]) - t)
+        assert (err <= tol).all(), (key, got[key], t, err / tol)
