@@ -451,12 +451,17 @@ __device__ inline float growth(float t)
 // DruckerPragerPlasticity::project (drucker_prager.rs:224-267 with :121-167).  Updates
 // F and the plastic state {det Fp, q, log volume gain} in place, given the left singular
 // vectors U and the singular values s of F; s comes back as the projected F's.  The
-// projected F = U s' V^T is F + U diag(s' / s - 1) U^T F: no right singular vectors, and the
-// rounding of U weighs only on the change (U s' V^T, and U diag(s' / s) U^T F more so, round
-// all of F anew at every plastic substep).
-__device__ inline void dp_project(const float *dp, float &pdet, float &q, float &lvg, m3 &F, const m3 &U, f3 &s)
+// projected F = U s' V^T is F + U diag(g) U^T F with the growths g = s' / s - 1: no right
+// singular vectors, and the rounding of U weighs only on the change (U s' V^T, and
+// U diag(s' / s) U^T F more so, round all of F anew at every plastic substep).  Where a
+// growth is beyond MAX_GROWTH the small part of F that grows is no better than the
+// rounding of its large one: true is returned, and the caller takes U s' V^T.  Against 64
+// bits, both forms in FP32: growths of 0.4 to 0.5 1.30e-7 (U s' V^T) and 1.24e-7, of 0.5 to
+// 0.6 1.28e-7 and 1.37e-7, of 0.8 to 1 1.3e-7 and 7e-7, of 2 to 4 1.8e-7 and 8e-7.
+constexpr float MAX_GROWTH = 0.5f;
+__device__ inline bool dp_project(const float *dp, float &pdet, float &q, float &lvg, m3 &F, const m3 &U, f3 &s)
 {
-    if (dp[4] == 0.0f) return;
+    if (dp[4] == 0.0f) return false;
     float alpha = dp_alpha(dp, q);
     const float d = 3.0f, inv_d3 = 1.0f / 3.0f;
     float lg = lvg * inv_d3;
@@ -465,29 +470,33 @@ __device__ inline void dp_project(const float *dp, float &pdet, float &q, float 
     float m = tr * inv_d3;
     f3 dev = mk3(strain.x - m, strain.y - m, strain.z - m);
     float shifted = tr - dp[6];
-    f3 g;       // growth of the singular values, s' / s - 1
+    f3 g, ns;   // growths of the singular values, and s'
     float dq;
     if (shifted > 0.0f || (dev.x == 0.0f && dev.y == 0.0f && dev.z == 0.0f)) {
         float e = __expf(dp[6] * inv_d3);
         g = mk3((e - s.x) * rcp_hw(s.x), (e - s.y) * rcp_hw(s.y), (e - s.z) * rcp_hw(s.z));
+        ns = mk3(e, e, e);
         dq = length(strain);
     } else {
         float dn = length(dev);
         float gamma = dn + (d * dp[4] + 2.0f * dp[5]) * rcp_hw(2.0f * dp[5]) * shifted * alpha;
-        if (gamma <= 0.0f) return;   // elastic: state and F unchanged
+        if (gamma <= 0.0f) return false;   // elastic: state and F unchanged
         // s' = exp(strain - k dev) with strain = log s + lg: s' / s = exp(lg - k dev).
         float k = gamma * rcp_hw(dn);
         g = mk3(growth(lg - dev.x * k), growth(lg - dev.y * k), growth(lg - dev.z * k));
+        ns = mk3(__expf(strain.x - dev.x * k), __expf(strain.y - dev.y * k), __expf(strain.z - dev.z * k));
         dq = gamma;
     }
-    const f3 ns = mk3(s.x + s.x * g.x, s.y + s.y * g.y, s.z + s.z * g.z);
+    const bool wide = !(fmaxf(fabsf(g.x), fmaxf(fabsf(g.y), fabsf(g.z))) <= MAX_GROWTH);
+    if (!wide) ns = mk3(s.x + s.x * g.x, s.y + s.y * g.y, s.z + s.z * g.z);
     float prev_det = s.x * s.y * s.z;
     float new_det = ns.x * ns.y * ns.z;
     pdet = pdet * prev_det * rcp_hw(new_det);
     lvg = lvg + __logf(prev_det) - __logf(new_det);
     q = q + dq;
-    F = F + mul(u_diag_ut(U, g), F);
+    if (!wide) F = F + mul(u_diag_ut(U, g), F);
     s = ns;
+    return wide;
 }
 
 // SnowPlasticity::project and hardening_factor (snow.rs:77-113), sp = {critical
@@ -495,10 +504,9 @@ __device__ inline void dp_project(const float *dp, float &pdet, float &q, float 
 // [1 - theta_c, 1 + theta_s], the removed volume change goes into the plastic
 // determinant (kept in [0.1, 4]) and the elastic moduli scale by
 // exp(hardening (1 - plastic det)).  Returns that factor; F and the plastic determinant
-// are updated in place and (U, s, V) is the SVD of the returned F.
-__device__ inline float snow_project(const float *sp, float &pdet, m3 &F, m3 &U, f3 &s, m3 &V)
+// are updated in place; (U, s, V) is the SVD of F before and after.
+__device__ inline float snow_project(const float *sp, float &pdet, m3 &F, const m3 &U, f3 &s, const m3 &V)
 {
-    svd3(F, U, s, V);
     if (sp[0] <= 0.0f && sp[1] <= 0.0f) return __expf(sp[2] * (1.0f - pdet));
     const float lo = 1.0f - sp[0], hi = 1.0f + sp[1];
     const f3 c = mk3(fminf(fmaxf(s.x, lo), hi), fminf(fmaxf(s.y, lo), hi), fminf(fmaxf(s.z, lo), hi));

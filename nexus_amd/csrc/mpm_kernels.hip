@@ -1985,22 +1985,34 @@ __device__ __forceinline__ void g2p_particle(const WorldDev &w, uint32_t pos, ui
                 tau = nh_stress(cls.w[0], cls.w[1], F);
             } else if (tag == 4u) {
                 tau = fluid_stress(cls.w, F, gradv);
-            } else if (tag == 5u) {
-                m3 U, V;
-                f3 sv;
-                const float hard = snow_project(cls.w + 1, ps0, F, U, sv, V);
-                tau = linear_stress_svd(cls.w[4] * hard, cls.w[5] * hard, U, sv);
-            } else if (tag <= 3u) {
-                // Corotated linear, and Drucker-Prager over either backbone: one copy of the SVD.
+            } else if (tag <= 5u) {
+                // Corotated linear, Drucker-Prager over either backbone, and snow: one copy of
+                // the SVD without V and one with it (snow, and a sand projection that is wide).
                 m3 U;
                 f3 sv;
-                svd3_us(F, U, sv);
                 const float *lame = cls.w;
-                if (tag != 0u) {
-                    dp_project(cls.w + 3, ps0, ps1, ps2, F, U, sv);
-                    lame += 10;
+                float hard = 1.0f;
+                bool wide = tag == 5u;
+                if (!wide) {
+                    svd3_us(F, U, sv);
+                    if (tag != 0u) {
+                        wide = dp_project(cls.w + 3, ps0, ps1, ps2, F, U, sv);
+                        lame += 10;
+                    }
                 }
-                tau = tag == 3u ? nh_stress(lame[0], lame[1], F) : linear_stress_svd(lame[0], lame[1], U, sv);
+                if (wide) {
+                    const f3 projected = sv;
+                    m3 V;
+                    svd3(F, U, sv, V);
+                    if (tag == 5u) {
+                        hard = snow_project(cls.w + 1, ps0, F, U, sv, V);
+                        lame += 4;
+                    } else {
+                        sv = projected;
+                        F = recompose(U, sv, V);
+                    }
+                }
+                tau = tag == 3u ? nh_stress(lame[0], lame[1], F) : linear_stress_svd(lame[0] * hard, lame[1] * hard, U, sv);
             }
             C = gradv * mass - tau * (vol0 * inv_d * dt);
             const bool nan_pos = npos.x != npos.x || npos.y != npos.y || npos.z != npos.z;
