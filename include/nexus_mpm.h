@@ -202,7 +202,8 @@ typedef struct {
  * Results do not depend on them (fixed-point P2G, per-particle and per-node stages), so
  * they can be tuned while a scene runs. */
 typedef struct {
-    uint32_t p2g_groups;      /* waves of the P2G kernel, at most (four to a workgroup) */
+    uint32_t p2g_groups;      /* waves of the P2G kernel, rounded up to 8 workgroups of four; a
+                               * small world launches fewer (one for 4 particles at most) */
     uint32_t p2g_block_cost;  /* per-block cost, in particles, of the P2G work split */
     uint32_t grid_groups;     /* workgroup cap of the grid-stride kernels (256 threads each) */
 } nxm_launch_config;

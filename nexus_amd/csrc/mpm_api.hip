@@ -894,7 +894,7 @@ class World {
         if (tune_on_ && !tuning_ && tuned_p_ && (p_in_ > 2 * tuned_p_ || 2 * p_in_ < tuned_p_)) start_tuning();
         const nxm_launch_config cfg = tuning_ ? tune_candidate() : cfg_;
         WorldDev w = view();
-        w.p2g_groups = p2g_workgroups(cfg.p2g_groups, p_in_);
+        w.p2g_groups = p2g_workgroups(cfg.p2g_groups, p_in_, any_cpic_);
         w.p2g_block_cost = cfg.p2g_block_cost;
         LaunchConfig lc{};
         lc.p_hint = p_in_;
@@ -2658,7 +2658,7 @@ nxm_status nxm_pipeline_step_noalloc(nxm_ctx *ctx, const nxm_noalloc_scene *scen
     const uint32_t b_total = h_total;
     const uint32_t p_cap = (n + 63u) & ~63u;
     const uint32_t cu = (uint32_t)ctx->num_cus;
-    const uint32_t p2g_groups = p2g_workgroups(cu * 32u, n);
+    const uint32_t p2g_groups = p2g_workgroups(cu * 32u, n, false);
     const uint32_t scan_stride = (h_total + SCAN_TILE - 1u) / SCAN_TILE + 2u;
     Carver c;
     const size_t o_arena0 = c.take<float>((size_t)NUM_PLANES * p_cap);
