@@ -1691,13 +1691,23 @@ class World {
         return NXM_OK;
     }
 
+    // A P2G candidate that launches what the one before it launched (a small world's limit,
+    // p2g_workgroups): left out, or noise would choose between the two.
+    bool repeats_launch(size_t idx) const
+    {
+        return tune_stage_ == 0 && p2g_workgroups(tune_cands_[idx].p2g_groups, p_in_, any_cpic_) ==
+                                       p2g_workgroups(tune_cands_[idx - 1].p2g_groups, p_in_, any_cpic_);
+    }
+
     // Called after each tuning substep; at the end of a stage reads the events (one
     // synchronization per stage) and moves to the next stage or finishes.
     nxm_status tune_advance()
     {
         if (++tune_rep_ < TUNE_REPS) return NXM_OK;
         tune_rep_ = 0;
-        if (++tune_idx_ < tune_cands_.size()) return NXM_OK;
+        do ++tune_idx_;
+        while (tune_idx_ < tune_cands_.size() && repeats_launch(tune_idx_));
+        if (tune_idx_ < tune_cands_.size()) return NXM_OK;
         HIP_TRY(hipStreamSynchronize(stream_));
         for (size_t k = 0; k < tune_used_; ++k) {
             float ms = 0.0f;
