@@ -1297,11 +1297,12 @@ __device__ __forceinline__ BlockScales block_scales(const WorldDev &w, uint32_t 
     return b;
 }
 
-// Scatter of one particle, by this lane as lane sel of the K that share it; returns the
-// staging regions it reaches (0: its base cell is not in the block).
+// Scatter of one particle, by this lane as lane sel of the K that share it (K = 0: as many as
+// lanes says, one copy of this for all of them); returns the staging regions it reaches (0:
+// its base cell is not in the block).
 template <int PART, int K>
 __device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *bad, const P2GIn &p, const BlockScales &b,
-                                            uint32_t sel, const uint32_t *naff, uint32_t pa)
+                                            uint32_t sel, const uint32_t *naff, uint32_t pa, uint32_t lanes = K)
 {
     const float h = b.h, ih = b.ih;
     // A sum that bounds |m v + C dpt|: finite and far below FLT_MAX, it says that the bound
@@ -1337,11 +1338,19 @@ __device__ __forceinline__ uint32_t p2g_one(unsigned long long *tile, uint32_t *
     q.hy = scaled(p.C.c1, hs);
     q.hz = scaled(p.C.c2, hs);
     q.mass = (double)p.m * (double)b.sm;
+    const int share = 27 / (int)lanes, q0 = (int)sel * share;
     if (!(sum < 0x1p120f) || !(fabsf(p.m) < 0x1p120f))
-        p2g_scatter_checked<PART>(tile, bad, q, (int)sel * (27 / K), ((int)sel + 1) * (27 / K),
-                                  ldexp(1.0, Fixed::BITS - log2_up(b.np)), naff, pa);
-    else
+        p2g_scatter_checked<PART>(tile, bad, q, q0, q0 + share, ldexp(1.0, Fixed::BITS - log2_up(b.np)), naff, pa);
+    else if constexpr (K != 0)
         p2g_scatter<PART, K>(tile, q, (int)sel, naff, pa);
+    else if (lanes == 1u)
+        p2g_scatter<PART, 1>(tile, q, 0, naff, pa);
+    else if (lanes == 3u)
+        p2g_scatter<PART, 3>(tile, q, (int)sel, naff, pa);
+    else if (lanes == 9u)
+        p2g_scatter<PART, 9>(tile, q, (int)sel, naff, pa);
+    else
+        p2g_scatter<PART, 27>(tile, q, (int)sel, naff, pa);
     return spill_mask(bx, by, bz);
 }
 
@@ -1405,11 +1414,15 @@ __device__ __forceinline__ uint32_t turn_lanes(const Turn &t)
     const uint32_t r = t.np - WAVE * t.c;
     return r <= 2u ? 27u : (r <= 7u ? 9u : (r <= 21u ? 3u : 1u));
 }
+// The particle of its turn that lane l shares with k - 1 others.
+__device__ __forceinline__ uint32_t shared_by(uint32_t l, uint32_t k)
+{
+    return k == 1u ? l : (k == 3u ? l / 3u : (k == 9u ? l / 9u : l / 27u));
+}
 __device__ __forceinline__ uint32_t turn_slot(const WorldDev &w, const Turn &t, uint32_t l)
 {
     if (t.np == 0u) return NONE;
-    const uint32_t k = turn_lanes(t);
-    const uint32_t i = WAVE * t.c + (k == 1u ? l : (k == 3u ? l / 3u : (k == 9u ? l / 9u : l / 27u)));
+    const uint32_t i = WAVE * t.c + shared_by(l, turn_lanes(t));
     return i < t.np ? w.perm[t.first + i] : NONE;
 }
 
@@ -1426,66 +1439,133 @@ __device__ __forceinline__ uint32_t team_touched(uint32_t *words, uint32_t l, ui
     return m;
 }
 
-// One block by a team, or (CPIC) by one wave: the crowded blocks, and the CPIC blocks with
-// nodes in reach of a collider.  Each wave takes its turns of 64 particles, the next one's
-// loads under the scatter of this one.
-template <bool CPIC, bool TEAM, int PART>
+// Scatter of a team's turns: a particle per lane, the next one's loads under the scatter of
+// this one.
+template <int PART>
 __device__ __forceinline__ uint32_t p2g_turns(const WorldDev &w, unsigned long long *tile, uint32_t *bad, const BlockScales &b,
                                               uint32_t first, uint32_t np, uint32_t l, const uint32_t *naff)
 {
+    constexpr uint32_t LANES = team_lanes<true>();
     uint32_t spill = 0u;
     auto slot_of = [&](uint32_t i) { return i < np ? w.perm[first + i] : NONE; };
     auto aff_of = [&](uint32_t i) { return PART != PART_ALL && i < np ? w.out.uplane(PAFF)[first + i] : 0u; };
-    uint32_t next = slot_of(l + team_lanes<TEAM>());
+    uint32_t next = slot_of(l + LANES);
     P2GLane q = p2g_fetch(w, slot_of(l));
-    for (uint32_t i = l; i - l % WAVE < np; i += team_lanes<TEAM>()) {
+    for (uint32_t i = l; i - l % WAVE < np; i += LANES) {
         const uint32_t pa = aff_of(i);
         const P2GLane now = q;
         q = p2g_fetch(w, next);
-        next = slot_of(i + 2 * team_lanes<TEAM>());
+        next = slot_of(i + 2 * LANES);
         if (now.on && (PART != PART_INCOMPATIBLE || (pa & 0xFFFFu) != 0u))
             spill |= p2g_one<PART, 1>(tile, bad, now.p, b, 0u, naff, pa);
     }
     return spill;
 }
 
-template <bool CPIC, bool TEAM>
-__device__ __forceinline__ void p2g_block(const WorldDev &w, uint32_t d, uint32_t np, const int4 v, uint32_t l,
-                                          unsigned long long *tile, uint32_t *bad, uint32_t *naff, const uint16_t *fdst,
-                                          uint32_t *words, bool &dirty)
+// One crowded block by a team.
+template <bool CPIC>
+__device__ __forceinline__ void p2g_team_block(const WorldDev &w, uint32_t d, uint32_t np, const int4 v,
+                                               unsigned long long *tile, uint32_t *bad, uint32_t *naff, const uint16_t *fdst,
+                                               uint32_t *words, bool &dirty)
 {
-    const uint32_t first = ld_uniform(w.bfirst + d);
+    const uint32_t l = threadIdx.x, first = ld_uniform(w.bfirst + d);
     const BlockScales b = block_scales(w, ld_uniform(w.bscene + d), v, ld_uniform(w.bprim + d), np);
     bool inc = false;
     if (CPIC && ld_uniform(w.breach + d)) {
-        for (uint32_t i = l; i < np; i += team_lanes<TEAM>())
-            inc |= (w.out.uplane(PAFF)[first + i] & 0xFFFFu) != 0u && (w.in.uplane(PFLAGS)[w.perm[first + i]] & FLAG_ENABLED);
+        for (uint32_t i = l; i < np; i += team_lanes<true>())
+            inc |= (w.out.uplane(PAFF)[first + i] & 0xFFFFu) != 0u;   // (a disabled one: a second tile of zeros)
         inc = __ballot(inc) != 0ull;
-        if (TEAM) {
-            if (l % WAVE == 0) words[l / WAVE] = inc ? 1u : 0u;
-            __syncthreads();
-            for (int k = 0; k < P2G_WAVES; ++k) inc |= words[k] != 0u;
-        }
+        if (l % WAVE == 0) words[l / WAVE] = inc ? 1u : 0u;
+        __syncthreads();
+        for (int k = 0; k < P2G_WAVES; ++k) inc |= words[k] != 0u;
     }
-    p2g_clear<TEAM>(tile, bad, l, dirty);
-    if (CPIC && inc) load_tile_affinity<TEAM>(w, d, naff, l);
-    team_sync<TEAM>();
+    p2g_clear<true>(tile, bad, l, dirty);
+    if (CPIC && inc) load_tile_affinity<true>(w, d, naff, l);
+    team_sync<true>();
     uint32_t spill;
-    if (CPIC && inc) spill = p2g_turns<CPIC, TEAM, PART_COMPATIBLE>(w, tile, bad, b, first, np, l, naff);
-    else spill = p2g_turns<CPIC, TEAM, PART_ALL>(w, tile, bad, b, first, np, l, naff);
-    const uint32_t touched = team_touched<TEAM>(words, l, spill);
-    p2g_flush<TEAM>(tile, bad, reinterpret_cast<float4 *>(w.stage), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+    if (CPIC && inc) spill = p2g_turns<PART_COMPATIBLE>(w, tile, bad, b, first, np, l, naff);
+    else spill = p2g_turns<PART_ALL>(w, tile, bad, b, first, np, l, naff);
+    const uint32_t touched = team_touched<true>(words, l, spill);
+    p2g_flush<true>(tile, bad, reinterpret_cast<float4 *>(w.stage), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
     dirty = touched == 0xFFu;
     if (CPIC && inc) {
         // Second pass: the incompatible contributions of the particles with affinity.
-        p2g_clear<TEAM>(tile, bad, l, dirty);
-        team_sync<TEAM>();
-        p2g_turns<CPIC, TEAM, PART_INCOMPATIBLE>(w, tile, bad, b, first, np, l, naff);
-        p2g_flush<TEAM>(tile, bad, reinterpret_cast<float4 *>(w.stage_i), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+        p2g_clear<true>(tile, bad, l, dirty);
+        team_sync<true>();
+        p2g_turns<PART_INCOMPATIBLE>(w, tile, bad, b, first, np, l, naff);
+        p2g_flush<true>(tile, bad, reinterpret_cast<float4 *>(w.stage_i), d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
         dirty = touched == 0xFFu;
     }
     unlink_untouched(w, d, touched, l);
     if (CPIC && l == 0) w.binc[d] = inc ? 1u : 0u;
+}
+
+// A particle of a turn and its affinity.
+struct ReachLane {
+    P2GLane q;
+    uint32_t pa, lanes, sel;
+};
+__device__ __forceinline__ ReachLane reach_lane(const WorldDev &w, const Turn &t, uint32_t l)
+{
+    ReachLane r;
+    r.lanes = turn_lanes(t);
+    const uint32_t share = shared_by(l, r.lanes), i = WAVE * t.c + share;
+    r.sel = l - r.lanes * share;
+    r.q = p2g_fetch(w, turn_slot(w, t, l));
+    r.pa = i < t.np ? w.out.uplane(PAFF)[t.first + i] : 0u;
+    return r;
+}
+template <int PART>
+__device__ __forceinline__ uint32_t reach_scatter(const ReachLane &r, unsigned long long *tile, uint32_t *bad,
+                                                  const BlockScales &b, const uint32_t *naff)
+{
+    if (!r.q.on || (PART == PART_INCOMPATIBLE && (r.pa & 0xFFFFu) == 0u)) return 0u;
+    return p2g_one<PART, 0>(tile, bad, r.q.p, b, r.sel, naff, r.pa, r.lanes);
+}
+
+// One CPIC block in reach of a collider by one wave, turn by turn; the particles of a block of
+// one turn are read once for both passes.  With one lane per particle in the last turn, the
+// affinities looked up through the slots first and the particles read anew for the second
+// pass, P2G of 60,000 particles in 17,612 blocks took 72.7 us (now 55.9), of 262,144 in
+// 6580 blocks 47.8 (45.9), of 1,048,576 in 21,764 blocks 114.6 (108.1).  Blocks of more than
+// 64 by a team: 60,000 in 2024 blocks 25.3 us instead of 31.6, but 1,048,576 152 instead
+// of 108.
+__device__ __forceinline__ void p2g_reach_block(const WorldDev &w, Turn t, uint32_t l, unsigned long long *tile, uint32_t *bad,
+                                                uint32_t *naff, const uint16_t *fdst, bool &dirty)
+{
+    ReachLane r = reach_lane(w, t, l);
+    const BlockScales b = block_scales(w, t.s, t.v, t.mass_code, t.np);
+    bool inc = (r.pa & 0xFFFFu) != 0u;   // (of a disabled particle alone: a second tile of zeros)
+    for (uint32_t i = WAVE + l; i < t.np; i += WAVE) inc |= (w.out.uplane(PAFF)[t.first + i] & 0xFFFFu) != 0u;
+    inc = __ballot(inc) != 0ull;
+    p2g_clear<false>(tile, bad, l, dirty);
+    if (inc) load_tile_affinity<false>(w, t.d, naff, l);
+    team_sync<false>();
+    uint32_t spill = 0u;
+    for (;;) {
+        spill |= inc ? reach_scatter<PART_COMPATIBLE>(r, tile, bad, b, naff) : reach_scatter<PART_ALL>(r, tile, bad, b, naff);
+        if (WAVE * ++t.c >= t.np) break;
+        r = reach_lane(w, t, l);
+    }
+    const uint32_t touched = wave_or_mask8(spill);
+    p2g_flush<false>(tile, bad, reinterpret_cast<float4 *>(w.stage), t.d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+    dirty = touched == 0xFFu;
+    if (inc) {
+        // Second pass: the incompatible contributions of the particles with affinity.
+        p2g_clear<false>(tile, bad, l, dirty);
+        team_sync<false>();
+        t.c = 0u;
+        if (t.np > (uint32_t)WAVE) r = reach_lane(w, t, l);
+        for (;;) {
+            reach_scatter<PART_INCOMPATIBLE>(r, tile, bad, b, naff);
+            if (WAVE * ++t.c >= t.np) break;
+            r = reach_lane(w, t, l);
+        }
+        p2g_flush<false>(tile, bad, reinterpret_cast<float4 *>(w.stage_i), t.d, b.smom, b.sm, l, touched, fdst, touched != 0xFFu);
+        dirty = touched == 0xFFu;
+    }
+    unlink_untouched(w, t.d, touched, l);
+    if (l == 0) w.binc[t.d] = inc ? 1u : 0u;
 }
 
 // Workgroups of P2G_WAVES waves, each with a cost-balanced range of blocks (p2g_split), the
@@ -1581,8 +1661,7 @@ __global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_
     }
     if (CPIC) {
         Turn t;
-        for (pop(1, t); t.np; pop(1, t))
-            p2g_block<CPIC, false>(w, t.d, t.np, t.v, l, tile, bad, naff, fdst, words, dirty);
+        for (pop(1, t); t.np; pop(1, t)) p2g_reach_block(w, t, l, tile, bad, naff, fdst, dirty);
     }
     bool first = true;
     dirty = true;
@@ -1593,7 +1672,7 @@ __global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_
         if (v.x == OVERFLOW_VID) continue;
         if (first) __syncthreads();   // the first wave has left its tile
         first = false;
-        p2g_block<CPIC, true>(w, d, np, v, threadIdx.x, tiles[0], bads[0], naffs[0], fdst, words, dirty);
+        p2g_team_block<CPIC>(w, d, np, v, tiles[0], bads[0], naffs[0], fdst, words, dirty);
     }
 }
 
