@@ -230,13 +230,15 @@ __device__ inline uint32_t particle_key(const WorldDev &w, uint32_t i, bool vali
     return key;
 }
 
-// The first lane of a run of neighbours in the wave with one (scene, key).
+// The first lane of a run of neighbours in the wave with one (scene, key).  Invalid lanes
+// are passed over: CPIC's contact particles, which another kernel keys, lie all through the
+// waves of the plain ones.
 __device__ inline bool run_starts(bool valid, uint32_t s, uint32_t key)
 {
-    const uint32_t pk = __shfl_up(key, 1, WAVE);
-    const uint32_t ps = __shfl_up(s, 1, WAVE);
-    const bool pv = __shfl_up((int)valid, 1, WAVE) != 0;
-    return valid && key != OVERFLOW_KEY && (lane_id() == 0 || !pv || pk != key || ps != s);
+    const uint64_t before = __ballot(valid) & (lanes_le(lane_id()) >> 1);
+    const int prev = before ? 63 - __clzll((long long)before) : 0;
+    const uint32_t pk = __shfl(key, prev, WAVE), ps = __shfl(s, prev, WAVE);
+    return valid && key != OVERFLOW_KEY && (!before || pk != key || ps != s);
 }
 
 // The key words of particle slot i (particle_key), its block's hash slot (to pslot[i]) and the wave's block insertions:
