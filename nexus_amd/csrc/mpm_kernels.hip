@@ -1576,6 +1576,9 @@ __device__ __forceinline__ void p2g_reach_block(const WorldDev &w, Turn t, uint3
 // then taken by all the waves together on one tile: a block's particles are one serial
 // chain otherwise (a block of 512 took 8 turns of 64, and a body of 32,768 particles at 8
 // per cell kept 64 waves of the chip busy).
+// Whether there are crowded ones the waves learn while they take the others, or each would
+// go through the range again while the workgroup holds its tiles (P2G of 1M sand with CPIC
+// 119.5 -> 113.7 us, of 2M clumped fluid 396 -> 387).
 // A wave works ahead: while it scatters one turn, the next turn's particles (of the same
 // block or the next) are being loaded and the slots of the one after are read, so that the
 // chain slot -> particle -> LDS adds of a block is not waited for.
@@ -1587,13 +1590,14 @@ __global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_
     __shared__ uint32_t bads[P2G_WAVES][BAD_ANY + 1];   // non-finite contributions; last word: any at all
     __shared__ uint32_t naffs[CPIC ? P2G_WAVES : 1][CPIC ? TILE_NODES : 1];
     __shared__ __align__(8) uint16_t fdst[TILE_NODES];
-    __shared__ uint32_t words[P2G_WAVES], queue[2];
+    __shared__ uint32_t words[P2G_WAVES], queue[2], crowded;
     const uint32_t G = gridDim.x, bx = blockIdx.x;
     const uint32_t g = (G % NUM_XCD == 0) ? (bx % NUM_XCD) * (G / NUM_XCD) + bx / NUM_XCD : bx;
     const uint32_t begin = ld_uniform(w.p2g_start + g), end = ld_uniform(w.p2g_start + g + 1);
     if (begin == end) return;
     load_flush_table(fdst, threadIdx.x);
     if (threadIdx.x < 2u) queue[threadIdx.x] = begin;
+    if (threadIdx.x == 0u) crowded = 0u;
     __syncthreads();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), l = lane_id();
     unsigned long long *tile = tiles[wave];
@@ -1609,6 +1613,7 @@ __global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_
             t.np = 0u;
             if (t.d >= end) return;
             const uint32_t np = ld_uniform(w.bnp + t.d);
+            if (np > TEAM_MIN) crowded = 1u;   // (by whichever lanes: the same value)
             if (np == 0u || np > TEAM_MIN) continue;
             t.v = ld_uniform(w.bvid + t.d);
             if (t.v.x == OVERFLOW_VID) continue;
@@ -1665,15 +1670,14 @@ __global__ void __launch_bounds__(P2G_WAVES * WAVE) __attribute__((amdgpu_waves_
         Turn t;
         for (pop(1, t); t.np; pop(1, t)) p2g_reach_block(w, t, l, tile, bad, naff, fdst, dirty);
     }
-    bool first = true;
+    __syncthreads();   // every block has been met, and the first wave has left its tile
+    if (crowded == 0u) return;
     dirty = true;
     for (uint32_t d = begin; d < end; ++d) {
         const uint32_t np = ld_uniform(w.bnp + d);
         if (np <= TEAM_MIN) continue;
         const int4 v = ld_uniform(w.bvid + d);
         if (v.x == OVERFLOW_VID) continue;
-        if (first) __syncthreads();   // the first wave has left its tile
-        first = false;
         p2g_team_block<CPIC>(w, d, np, v, tiles[0], bads[0], naffs[0], fdst, words, dirty);
     }
 }
