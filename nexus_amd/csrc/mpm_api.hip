@@ -24,6 +24,7 @@
 
 #include "../../include/nexus_mpm.h"
 #include "mpm_kernels.h"
+#include "pinned_pool.h"
 
 namespace nxm {
 
@@ -84,76 +85,6 @@ struct DevBuf {
 
 using namespace nxm;
 
-// Pinned host chunks shared by the threads of one context: a scene staged for upload on
-// one thread (nxm_scene_stage_upload) holds a chunk until the thread stepping its world
-// queues the copies; the chunk is reused once those copies have executed.  Readbacks have
-// chunks of their own, given back when nothing is queued on them: they need no event, and so
-// never ask for one last recorded on a stream that has gone or is being captured.
-struct PinnedPool {
-    struct Chunk {
-        char *p = nullptr;
-        size_t n = 0;
-        hipEvent_t ev = nullptr;   // null: a readback's
-        bool held = false;
-    };
-    std::mutex mu;
-    std::vector<Chunk> chunks;
-
-    // The smallest free chunk of at least `bytes` whose last copies have executed.
-    hipError_t take(size_t bytes, int *idx, char **out, bool readback = false)
-    {
-        std::lock_guard<std::mutex> g(mu);
-        int best = -1;
-        for (int k = 0; k < (int)chunks.size(); ++k) {
-            Chunk &c = chunks[k];
-            if (c.held || c.n < bytes || readback != (c.ev == nullptr)) continue;
-            if (best >= 0 && chunks[best].n <= c.n) continue;
-            const hipError_t q = readback ? hipSuccess : hipEventQuery(c.ev);
-            if (q == hipErrorNotReady) continue;
-            if (q != hipSuccess) return q;
-            best = k;
-        }
-        if (best < 0) {
-            Chunk c;
-            c.n = std::max<size_t>(bytes, (size_t)1 << 20);
-            hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&c.p), c.n, hipHostMallocDefault);
-            if (e != hipSuccess) return e;
-            if (!readback) e = hipEventCreate(&c.ev);
-            if (e != hipSuccess) { (void)hipHostFree(c.p); return e; }
-            chunks.push_back(c);
-            best = (int)chunks.size() - 1;
-        }
-        chunks[best].held = true;
-        *idx = best;
-        *out = chunks[best].p;
-        return hipSuccess;
-    }
-    // Gives the chunk back; with a stream, reusable once the work queued so far has run.
-    hipError_t give(int idx, hipStream_t st)
-    {
-        std::lock_guard<std::mutex> g(mu);
-        Chunk &c = chunks[idx];
-        hipError_t e = st ? hipEventRecord(c.ev, st) : hipSuccess;
-        c.held = false;
-        return e;
-    }
-    char *ptr(int idx)
-    {
-        std::lock_guard<std::mutex> g(mu);
-        return chunks[idx].p;
-    }
-    ~PinnedPool()
-    {
-        for (auto &c : chunks) {
-            if (c.ev) {
-                (void)hipEventSynchronize(c.ev);
-                (void)hipEventDestroy(c.ev);
-            }
-            (void)hipHostFree(c.p);
-        }
-    }
-};
-
 struct nxm_ctx {
     int device = 0;
     int num_cus = 256;
@@ -162,7 +93,7 @@ struct nxm_ctx {
     // until the last of them is destroyed.
     std::atomic<int> refs{0};
     std::atomic<bool> closed{false};
-    PinnedPool pool;
+    std::shared_ptr<PinnedPool> pool = std::make_shared<PinnedPool>();
 };
 
 // Scratch of nxm_pipeline_step_noalloc: one per GPU (each device holds its own copy of
@@ -502,7 +433,7 @@ struct nxm_scene {
     uint32_t dev_col_start = 0xFFFFFFFFu;
     bool cols_host = true;
     // Particles packed ahead of the next upload (nxm_scene_stage_upload): a chunk of the
-    // context's pinned pool in arena-plane layout, flags without the world slot.
+    // context's pinned pool in the arena's quads, flags without the world slot.
     int staged_chunk = -1;
     size_t staged_n = 0;
     std::vector<SceneRange> ranges;     // particle ranges in the world's input arena
@@ -559,6 +490,7 @@ class World {
     {
         if (stream_) {
             (void)hipStreamSynchronize(stream_);
+            uploads_.drain();
             drop_graphs();
             for (auto &e : ev_) (void)hipEventDestroy(e);
             for (auto &e : tune_ev_) (void)hipEventDestroy(e);
@@ -599,6 +531,7 @@ class World {
     {
         HIP_TRY(hipSetDevice(ctx_->device));
         HIP_TRY(hipStreamSynchronize(stream_));
+        uploads_.drain();
         return collect_errors();
     }
 
@@ -659,14 +592,16 @@ class World {
             if (first == 0 && count == sc->staged_n) {
                 // Packed by nxm_scene_stage_upload: add the world slot to the flags and queue.
                 const int k = sc->staged_chunk;
-                float *f = reinterpret_cast<float *>(sc->ctx->pool.ptr(k));
+                float *f = reinterpret_cast<float *>(sc->ctx->pool->ptr(k));
                 uint32_t *uf = reinterpret_cast<uint32_t *>(f) + PFLAGS;   // in the first quad
                 const uint32_t sbits = sc->slot << 16;
                 for (size_t i = 0; i < count; ++i) uf[4 * i] |= sbits;
                 const uint32_t at = p_in_;
-                HIP_TRY(put_quads(f, at, count));
+                const hipError_t e = put_quads(f, at, count);
+                if (e != hipSuccess) (void)hipStreamSynchronize(stream_);   // nothing still reads the chunk
+                HIP_TRY(e);
                 sc->staged_chunk = -1;
-                HIP_TRY(sc->ctx->pool.give(k, stream_));
+                HIP_TRY(uploads_.add(sc->ctx->pool, k, stream_));
                 sc->ranges.push_back(SceneRange{at, (uint32_t)count});
                 p_in_ += (uint32_t)count;
                 pin_dirty_ = true;
@@ -674,7 +609,7 @@ class World {
             }
             const int k = sc->staged_chunk;   // stale: the particles changed since
             sc->staged_chunk = -1;
-            HIP_TRY(sc->ctx->pool.give(k, nullptr));
+            sc->ctx->pool->give(k);
         }
         char *stage = nullptr;
         size_t ci = 0;
@@ -798,10 +733,10 @@ class World {
         const size_t nslots = std::min(slots_.size(), ctr_.n);
         int held = -1;
         char *pin = nullptr;
-        HIP_TRY(ctx_->pool.take(2 * READ_CHUNK + MAX_SCENES * sizeof(SceneCtr), &held, &pin, true));
+        HIP_TRY(ctx_->pool->take(2 * READ_CHUNK + MAX_SCENES * sizeof(SceneCtr), &held, &pin));
         nxm_status st = copy_through(pin, reinterpret_cast<const char *>(dev), total, parts, nslots);
         if (st != NXM_OK) (void)hipStreamSynchronize(stream_);   // nothing still writes the chunk
-        HIP_TRY(ctx_->pool.give(held, nullptr));
+        ctx_->pool->give(held);
         return st;
     }
 
@@ -881,6 +816,7 @@ class World {
     nxm_status step(nxm_stage_times *times)
     {
         HIP_TRY(hipSetDevice(ctx_->device));
+        HIP_TRY(uploads_.poll());
         if (dirty_) {
             nxm_status st = rebuild_tables();
             if (st != NXM_OK) return st;
@@ -1786,6 +1722,7 @@ class World {
     std::vector<size_t> tune_slot_;
     std::vector<hipEvent_t> tune_ev_;
     std::vector<PinnedChunk> pins_;
+    PendingUploads uploads_;
     static constexpr size_t READ_CHUNK = (size_t)4 << 20;
     hipEvent_t read_ev_[2] = {};
     DevBuf<float4> read_palette_;
@@ -1909,7 +1846,7 @@ static nxm_status ensure_own_world(nxm_scene *sc)
 static void drop_staged(nxm_scene *sc)
 {
     if (sc->staged_chunk < 0) return;
-    (void)sc->ctx->pool.give(sc->staged_chunk, nullptr);
+    sc->ctx->pool->give(sc->staged_chunk);
     sc->staged_chunk = -1;
 }
 
@@ -2086,7 +2023,7 @@ void nxm_scene_destroy(nxm_scene *sc)
     sc->world = nullptr;
     sc->own.reset();
     nxm_ctx *ctx = sc->ctx;
-    if (sc->staged_chunk >= 0) (void)ctx->pool.give(sc->staged_chunk, nullptr);
+    if (sc->staged_chunk >= 0) ctx->pool->give(sc->staged_chunk);
     delete sc;
     ctx_release(ctx);
 }
@@ -2098,13 +2035,13 @@ nxm_status nxm_scene_stage_upload(nxm_scene *sc)
     const HostParticles &hp = sc->hp;
     const size_t n = hp.n;
     if (sc->staged_chunk >= 0) {
-        (void)sc->ctx->pool.give(sc->staged_chunk, nullptr);
+        sc->ctx->pool->give(sc->staged_chunk);
         sc->staged_chunk = -1;
     }
     if (n == 0) return NXM_OK;
     int k = -1;
     char *buf = nullptr;
-    HIP_TRY(sc->ctx->pool.take((size_t)NUM_PLANES * n * 4, &k, &buf));
+    HIP_TRY(sc->ctx->pool->take((size_t)NUM_PLANES * n * 4, &k, &buf));
     float *f = reinterpret_cast<float *>(buf);
     pack_particles(hp, 0, n, 0u, f);
     sc->staged_chunk = k;
