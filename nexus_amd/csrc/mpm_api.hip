@@ -834,7 +834,8 @@ class World {
         w.p2g_block_cost = cfg.p2g_block_cost;
         LaunchConfig lc{};
         lc.p_hint = p_in_;
-        lc.persistent_blocks = (int)cfg.grid_groups;
+        // (2^24 workgroups of 256 threads cover every particle and slot: a larger cap means none)
+        lc.persistent_blocks = (int)std::min<uint32_t>(cfg.grid_groups, 1u << 24);
         lc.p2g_blocks = (int)w.p2g_groups;
         hipEvent_t *evs = times ? ev_ : nullptr;
         if (!times && profiling_ && profile_seen_++ % profile_every_ == 0) {
