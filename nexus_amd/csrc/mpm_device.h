@@ -146,15 +146,6 @@ __device__ __forceinline__ T ld_uniform(const T *p)
     return r;
 }
 
-// ld_uniform where SCALAR holds (a kernel variant with scalar registers to spare), else a
-// plain load.
-template <bool SCALAR, class T>
-__device__ __forceinline__ T ld_maybe_uniform(const T *p)
-{
-    if constexpr (SCALAR) return ld_uniform(p);
-    else return *p;
-}
-
 struct ColliderDev {
     float he[3];
     float q[4];

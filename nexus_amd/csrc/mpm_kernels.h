@@ -151,7 +151,7 @@ void launch_canonical(const WorldDev &w, const Arena &prev, uint32_t *pcell, uin
 constexpr int NOALLOC_MAX_CLASSES = 16;
 constexpr int NOALLOC_MAX_COLLIDERS = 16;
 // A cuboid of that path: ColliderDev's leading body fields (the nxm_cuboid words) and its
-// bounding radius; k_noalloc_tables completes the record.
+// bounding radius; k_noalloc_setup completes the record.
 constexpr int COLLIDER_BODY_WORDS = 24;
 static_assert(offsetof(ColliderDev, shape) == COLLIDER_BODY_WORDS * sizeof(float), "body words lead ColliderDev");
 struct NoallocCuboid {

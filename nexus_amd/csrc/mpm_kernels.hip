@@ -306,9 +306,9 @@ __device__ inline void mark_overflow_slots(const WorldDev &w)
 // set in LDS.  A block new to the set is looked up, and one found marked is left alone (keys
 // and marks only ever turn on, so a stale line can only send a workgroup the long way); the
 // workgroup whose atomic marks it inserts its 7 neighbours.  Against eight insertions per
-// run, with 256 threads: 1M particles in random order 496 -> 307 us, 2M in clumps 1322 -> 111.
-// (Groups of 1024 and of 256: 111-161 us and 165 for the clumps, a call of 1000 particles
-// 1-2 us slower with 1024.)
+// run, with 256 threads: 1M particles in random order 496 -> 326 us, 2M in clumps 1322 -> 161.
+// (Groups of 256 and 1024 took as long for the clumps, and a call of 1000 particles 1-2 us
+// more with 1024.)
 constexpr int KEY_GROUP = 512;
 struct KeySet {
     static constexpr uint32_t SIZE = 2 * KEY_GROUP;
@@ -1022,9 +1022,9 @@ struct Fixed {
     // can stand in t): three double operations and one 32-bit sum.  Doubles run at
     // the rate of floats here.  The product is exact before each rounding, so an integer
     // depends on a and w alone.
-    // One rounding to a unit of 2^(e - 51) takes a third of the double operations (P2G of 1M
-    // sand 78 us against 83, of 2M clumped fluid 400 against 421), but small contributions,
-    // such as the mass at the rim of a stencil, then have up to 11 bits less.
+    // One rounding to a unit of 2^(e - 51) takes a third of the double operations (P2G 3-6 %
+    // less: 1M sand 78 us against 82.6), but small contributions, such as the mass at the rim
+    // of a stencil, then have up to 11 bits less.
     static constexpr int BITS = 62;
     static constexpr double ONE = (double)0x43380000u * 0x1p32, T = 0x1.8p84 - ONE, R = 0x1.8p52;
     __device__ static word of(double a, double w)
@@ -2321,8 +2321,7 @@ __device__ inline void prepare_next_sort(const WorldDev &w)
 
 // One thread per sorted particle, nodes read from the grid: the launch (g2p_groups) gives
 // every workgroup at most g2p_threads positions, and a thread takes at most one, so no loop keeps
-// the arenas' 60-odd plane addresses live in scalar registers (they spilled to vector
-// lanes and were read back for every particle).  In CPIC worlds this kernel takes the
+// the addresses of both arenas' quads and of the tables live in scalar registers.  In CPIC worlds this kernel takes the
 // plain particles and k_g2p_contact the contact ones, so that the contact code does not
 // weigh on the register budget of the common path.  Then the new positions give
 // the next substep's block keys and insertions (touch_keys): the output arena is the next
