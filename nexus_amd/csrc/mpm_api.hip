@@ -830,7 +830,7 @@ class World {
         if (tune_on_ && !tuning_ && tuned_p_ && (p_in_ > 2 * tuned_p_ || 2 * p_in_ < tuned_p_)) start_tuning();
         const nxm_launch_config cfg = tuning_ ? tune_candidate() : cfg_;
         WorldDev w = view();
-        w.p2g_groups = p2g_workgroups(cfg.p2g_groups, p_in_, any_cpic_);
+        w.p2g_groups = p2g_workgroups(cfg.p2g_groups, p_in_, !any_cpic_);
         w.p2g_block_cost = cfg.p2g_block_cost;
         LaunchConfig lc{};
         lc.p_hint = p_in_;
@@ -1634,8 +1634,8 @@ class World {
     // p2g_workgroups): left out, or noise would choose between the two.
     bool repeats_launch(size_t idx) const
     {
-        return tune_stage_ == 0 && p2g_workgroups(tune_cands_[idx].p2g_groups, p_in_, any_cpic_) ==
-                                       p2g_workgroups(tune_cands_[idx - 1].p2g_groups, p_in_, any_cpic_);
+        return tune_stage_ == 0 && p2g_workgroups(tune_cands_[idx].p2g_groups, p_in_, !any_cpic_) ==
+                                       p2g_workgroups(tune_cands_[idx - 1].p2g_groups, p_in_, !any_cpic_);
     }
 
     // Called after each tuning substep; at the end of a stage reads the events (one

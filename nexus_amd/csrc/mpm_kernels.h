@@ -91,7 +91,7 @@ constexpr uint32_t ORDER_EVERY = 16;
 // one-wave groups are asked for, in whole rounds of the 8 XCDs.
 // - A block with particles holds 4 or more in most scenes, so more waves than p / 4 find
 //   no block (1000 particles: P2G 20 us with 8192 waves, 12 with 256).
-// - Without CPIC, three workgroups on each of the 256 CUs up to 2^17 particles and four up
+// - With resident (worlds without CPIC), three workgroups on each of the 256 CUs up to 2^17 particles and four up
 //   to 2^18: a CU holds four (their registers), so that these all run at once, with several
 //   blocks each for their waves.  Substeps with 3072, 4096 and 8192 waves: sand of 50,000
 //   particles 57.5, 58.5 and 59.6 us, of 100,003 67.8, 68.1 and 71.8, of 200,000 89.9, 89.3
@@ -99,15 +99,17 @@ constexpr uint32_t ORDER_EVERY = 16;
 //   65,536 65.6, 67.6 and 66.2, of 200,000 82.9, 84.7 and 85.6; cubes of 97,336 72.7, 72.9 and
 //   74.0, of 195,112 89.3, 91.2 and 89.8.  Above, more groups even out the blocks' costs: a
 //   cube of 300,763 104.4, 105.5 and 103.9, fluid of 1,000,000 443, 417 and 412; so they do
-//   for CPIC, whose blocks at a collider take two passes (262,144: 180, 171 and 170).
+//   for CPIC, whose blocks at a collider take two passes (262,144: 180, 171 and 170), and
+//   for the call without allocation, whose particles lie in the caller's order (120,001
+//   sand 117 and 110, 30,000 88.3 and 86.7; 60,000 100 and 100).
 constexpr int P2G_WAVES = 4;
 constexpr uint32_t CUS = 256;
-inline uint32_t p2g_workgroups(uint32_t groups, uint64_t p, bool cpic)
+inline uint32_t p2g_workgroups(uint32_t groups, uint64_t p, bool resident)
 {
     uint64_t waves = groups < p / 4 ? groups : p / 4;
-    if (!cpic && p <= 1u << 18) {
-        const uint64_t resident = (p <= 1u << 17 ? 3 : 4) * P2G_WAVES * CUS;
-        if (waves > resident) waves = resident;
+    if (resident && p <= 1u << 18) {
+        const uint64_t once = (p <= 1u << 17 ? 3 : 4) * P2G_WAVES * CUS;
+        if (waves > once) waves = once;
     }
     const uint64_t workgroups = (waves + P2G_WAVES - 1) / P2G_WAVES;
     return (uint32_t)(workgroups ? (workgroups + 7) / 8 * 8 : 8);
