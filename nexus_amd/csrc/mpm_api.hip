@@ -1590,8 +1590,8 @@ class World {
     {
         const uint32_t cu = (uint32_t)ctx_->num_cus;
         std::vector<nxm_launch_config> c;
-        // (P2G of CPIC sand of 1M with 32, 64 and 128: 124, 120 and 151 us; fluid of 2M 415,
-        // 396 and 399, of 8M with 32, 64, 256 and 512: 1549, 1380, 1318 and 1385)
+        // (P2G of CPIC sand of 1M with 32, 64 and 128: 116, 107 and 138 us; fluid of 2M 338, 315
+        // and 310, of 8M with 32, 64, 256 and 512: 1254, 1140, 1067 and 1089)
         if (stage == 0) for (uint32_t k : {32u, 64u, 256u}) c.push_back({cu * k, b.p2g_block_cost, b.grid_groups});
         if (stage == 1) for (uint32_t k : {4u, 16u, 64u}) c.push_back({b.p2g_groups, k, b.grid_groups});
         if (stage == 2) for (uint32_t k : {4u, 8u, 16u, 32u, 64u}) c.push_back({b.p2g_groups, b.p2g_block_cost, cu * k});

@@ -91,17 +91,17 @@ constexpr uint32_t ORDER_EVERY = 16;
 // one-wave groups are asked for, in whole rounds of the 8 XCDs.
 // - A block with particles holds 4 or more in most scenes, so more waves than p / 4 find
 //   no block (1000 particles: P2G 20 us with 8192 waves, 12 with 256).
-// - With resident (worlds without CPIC), three workgroups on each of the 256 CUs up to 2^17 particles and four up
-//   to 2^18: a CU holds four (their registers), so that these all run at once, with several
-//   blocks each for their waves.  Substeps with 3072, 4096 and 8192 waves: sand of 50,000
-//   particles 57.5, 58.5 and 59.6 us, of 100,003 67.8, 68.1 and 71.8, of 200,000 89.9, 89.3
-//   and 91.2; fluid of 50,000 70.9, 70.4 and 73.3, of 200,000 131, 125.6 and 131.8; snow of
-//   65,536 65.6, 67.6 and 66.2, of 200,000 82.9, 84.7 and 85.6; cubes of 97,336 72.7, 72.9 and
-//   74.0, of 195,112 89.3, 91.2 and 89.8.  Above, more groups even out the blocks' costs: a
-//   cube of 300,763 104.4, 105.5 and 103.9, fluid of 1,000,000 443, 417 and 412; so they do
-//   for CPIC, whose blocks at a collider take two passes (262,144: 180, 171 and 170), and
-//   for the call without allocation, whose particles lie in the caller's order (120,001
-//   sand 117 and 110, 30,000 88.3 and 86.7; 60,000 100 and 100).
+// - With resident (worlds without CPIC), three workgroups on each of the 256 CUs up to 2^17
+//   particles and four up to 2^18: a CU holds four (their registers), so that these all run
+//   at once, with several blocks each for their waves.  Substeps with 3072, 4096 and 8192
+//   waves: sand of 50,000 particles 57.0, 58.0 and 59.1 us, of 100,003 66.0, 66.4 and 71.4,
+//   of 200,000 87.4, 85.9 and 88.1; fluid of 50,000 67.5, 67.2 and 70.1, of 200,000 126,
+//   122 and 128; snow of 65,536 66.0, 68.4 and 66.8, of 200,000 83.3, 85.5 and 86.2; cubes of
+//   97,336 71.6, 72.2 and 73.6, of 195,112 89.0, 91.2 and 90.3.  Above, more groups even out
+//   the blocks' costs: a cube of 300,763 103.0, 104.0 and 102.4, fluid of 1,000,000 406, 387
+//   and 380; so they do for CPIC, whose blocks at a collider take two passes (262,144 in
+//   17,642 blocks 224, 213 and 209), and for the call without allocation, whose particles
+//   lie in the caller's order (120,001 sand 117 with 3072 and 110).
 constexpr int P2G_WAVES = 4;
 constexpr uint32_t CUS = 256;
 inline uint32_t p2g_workgroups(uint32_t groups, uint64_t p, bool resident)
